@@ -329,7 +329,11 @@ class StreamDecoder:
     @torch.no_grad()
     def _capture(self) -> None:
         """One graph per bucket, on the decoder stream; each program runs once eagerly first (every launch
-        validated), then is recorded. The state is reset afterwards (the runs advanced the dummy rows only)."""
+        validated), then is recorded. The state is reset afterwards (the runs advanced the dummy rows only). The runs
+        read the slots' state and the weights, which the constructor filled on the current stream: the decoder stream
+        waits for those fills (behind other queued work they may be far from done, and a token or an active row read
+        before its fill is an arbitrary index)."""
+        self.stream.wait_stream(torch.cuda.current_stream(self.device))
         with torch.cuda.stream(self.stream):
             for b in reversed(self.buckets):
                 self._run(b)

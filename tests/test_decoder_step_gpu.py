@@ -363,3 +363,33 @@ def test_fused_step_matches_unfused(int8, gpu):
         # the fused pick writes the stepped slots' end flags to the host itself; the unfused step copies them
         assert np.array_equal(a.flags.numpy()[slots], b.flags.numpy()[slots])
         assert np.array_equal(a.flags.numpy()[slots], a.finished.cpu().numpy()[slots])
+
+
+def test_decoder_built_behind_queued_work(gpu):
+    """A decoder constructed while the current stream still has queued work: the runs that precede the recording wait
+    for the fills of the decoder's state (tokens, active rows), which are queued behind that work. Its steps equal
+    those of a decoder built on an idle GPU, bit for bit."""
+    from kernels.stream_decoder import StreamDecoder
+
+    model = make_decoder(hidden=512, heads=4, layers=1, ffn=512, vocab=512, seed=15, device=gpu, dtype=torch.bfloat16)
+    kw = dict(slots=4, max_new_tokens=8, max_prompt=4, buckets=(4,), int8=False, frames=8)
+    torch.cuda.synchronize()
+    idle = StreamDecoder(model, **kw)
+    a = torch.randn(4096, 4096, device=gpu)
+    torch.cuda.synchronize()
+    for _ in range(20):  # some milliseconds of work ahead of the fills
+        a = torch.tanh(a @ a)
+    busy = StreamDecoder(model, **kw)
+    torch.cuda.synchronize()
+    mem = torch.randn(16, 512, generator=torch.Generator().manual_seed(16)).to(torch.bfloat16).to(gpu)
+    slots, lengths = [0, 1, 2], [8, 3, 5]
+    prompts = [torch.tensor([5 + i, 9]) for i in slots]
+    for d in (idle, busy):
+        d.fill_cross(mem, lengths, slots)
+        torch.cuda.synchronize()
+        d.admit(slots, prompts, lengths)
+        b = d.set_active(slots)
+        d.step(b, 4)
+    torch.cuda.synchronize()
+    for name in ("logits", "tok", "pos", "out", "self_k", "self_v"):
+        assert torch.equal(getattr(idle, name), getattr(busy, name)), name
