@@ -14,6 +14,8 @@
 #include "cohere_hip.h"
 #include "common.h"
 
+#include <algorithm>
+
 namespace {
 
 constexpr int NFFT = 512, HOP = 160, BINS = NFFT / 2 + 1, MELS = 128, NZ = NFFT / 2;
@@ -27,6 +29,9 @@ DEVI Cx csub(Cx a, Cx b) { return {a.re - b.re, a.im - b.im}; }
 DEVI Cx cmul(Cx a, Cx b) { return {a.re * b.re - a.im * b.im, a.re * b.im + a.im * b.re}; }
 DEVI Cx mul_mi(Cx a) { return {a.im, -a.re}; }  // a * (-i)
 
+// this wave's LDS accesses so far are done, and none after is moved before
+DEVI void wave_lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+
 // the piece holding flat frame f: the last p with frame_start[p] <= f
 DEVI int piece_of(const int64_t* frame_start, int pieces, int64_t f) {
   int lo = 0, hi = pieces - 1;
@@ -38,143 +43,246 @@ DEVI int piece_of(const int64_t* frame_start, int pieces, int64_t f) {
   return lo;
 }
 
+// Bound by vector-instruction issue: about 1000 instructions a frame, 4 cycles each (12,800 frames: 21 us of issue over
+// the 1024 SIMDs, 28 us measured, 29 with one frame per wave, tables per frame and a branch around each sample load).
+// A wave takes `per_wave` consecutive frames, so that the twiddle table (computed in double) and the mel weights in LDS
+// are made once for FPW * per_wave frames; the samples of its next frame are loaded while one is transformed. Its
+// FFT buffers are its own: between the passes it waits for its own LDS accesses only.
+constexpr int MTAPS = 16;  // a band's first weights, held in LDS (the extractor's bands have at most 13)
 __global__ void __launch_bounds__(FPW * 64) logmel_kernel(const float* __restrict__ x, const int64_t* __restrict__ meta,
-                                                          int pieces, int64_t total_frames,
+                                                          int pieces, int64_t total_frames, int per_wave,
                                                           const float* __restrict__ window,
                                                           const float* __restrict__ mel, const int* __restrict__ band,
                                                           float preemph, float* __restrict__ logmel) {
   __shared__ Cx tw[NFFT];            // e^{-2 pi i k / 512}
   __shared__ Cx buf[FPW][2][NZ];     // Stockham ping-pong, per wave
   __shared__ float power[FPW][BINS + 3];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  __shared__ float mw[MTAPS][MELS];
+  const int lane = threadIdx.x & 63, w = wave_id();
+  const int64_t* sample_start = meta;
+  const int64_t* lens = meta + pieces;
+  const int64_t* frame_start = meta + 2 * pieces;
+  const int64_t first = ((int64_t)blockIdx.x * FPW + w) * per_wave, end = min(first + per_wave, total_frames);
+
+  // lane j holds z[j + 64 r] = frame[2 (j + 64 r)] + i frame[2 (j + 64 r) + 1], r = 0..3; frame[j] is sample
+  // 160 t - 256 + j of the piece, pre-emphasised (x[s] - p x[s-1], the product rounded first), zero outside it, times
+  // the centred window
+  int p = first < end ? piece_of(frame_start, pieces, first) : 0;
+  // samples j - 1, j, j + 1 of the lane's four pairs; the frame's samples [jlo, jhi) are the piece's, the others load
+  // one of these (a guarded load would be a branch, and each branch a memory round trip of its own)
+  float raw[4][3];
+  int nlo = 0, nhi = 0, n0 = -1;
+  auto load = [&](int64_t f) {
+    while (p + 1 < pieces && frame_start[p + 1] <= f) ++p;  // pieces without frames are passed over
+    const int64_t s0 = (f - frame_start[p]) * HOP - NFFT / 2, n = lens[p];  // the frame's first sample
+    nlo = (int)min(max(-s0, (int64_t)0), (int64_t)NFFT);
+    nhi = (int)min(max(n - s0, (int64_t)0), (int64_t)NFFT);
+    n0 = s0 <= 0 ? nlo : -1;  // sample 0's place in the frame
+    const bool has = n > 0 && nhi > 0 && nlo < NFFT;
+    const int from = s0 > 0 ? -1 : nlo, to = nhi - 1;  // readable: [from, to]
+    const float* xp = x + sample_start[p] + s0;
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const int j = 2 * (lane + 64 * r) - 1 + k;
+        raw[r][k] = has ? xp[min(max(j, from), to)] : 0.f;
+      }
+  };
+  if (first < end) load(first);
+  float win[4][2];
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int k = 0; k < 2; ++k) win[r][k] = window[2 * (lane + 64 * r) + k];
+  int k0[2], k1[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    k0[h] = band[2 * (lane + 64 * h)];
+    k1[h] = band[2 * (lane + 64 * h) + 1];
+  }
+  for (int i = threadIdx.x; i < MTAPS * MELS; i += FPW * 64) {
+    const int m = i % MELS, k = band[2 * m] + i / MELS;
+    mw[i / MELS][m] = k < band[2 * m + 1] ? mel[(int64_t)m * BINS + k] : 0.f;
+  }
   for (int k = threadIdx.x; k < NFFT; k += FPW * 64) {
     double s, c;
     sincospi(-(double)k / 256.0, &s, &c);
     tw[k] = {(float)c, (float)s};
   }
-  const int64_t f = (int64_t)blockIdx.x * FPW + w;
-  const bool live = f < total_frames;
-  const int64_t* sample_start = meta;
-  const int64_t* lens = meta + pieces;
-  const int64_t* frame_start = meta + 2 * pieces;
+  __syncthreads();  // twiddle table and mel weights
 
-  // lane j holds z[j + 64 r] = frame[2 (j + 64 r)] + i frame[2 (j + 64 r) + 1], r = 0..3; frame[j] is sample
-  // 160 t - 256 + j of the piece, pre-emphasised (x[s] - p x[s-1], the product rounded first), zero outside it, times
-  // the centred window
-  Cx v[4];
-  if (live) {
-    const int p = piece_of(frame_start, pieces, f);
-    const int64_t t = f - frame_start[p];
-    const float* xp = x + sample_start[p];
-    const int64_t n = lens[p];
-    auto sample = [&](int j) {
-      const int64_t s = t * HOP - NFFT / 2 + j;
-      float e = 0.f;
-      if (s >= 0 && s < n) e = s == 0 ? xp[0] : __fsub_rn(xp[s], __fmul_rn(preemph, xp[s - 1]));
-      return __fmul_rn(e, window[j]);
-    };
+  // the lane's twiddles of the passes and of the split: the same for every frame
+  Cx wp[3][3], ws[4];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const int Ns = 4 << (2 * i);
+#pragma unroll
+    for (int r = 1; r < 4; ++r) wp[i][r - 1] = tw[(r * (lane % Ns) * (128 / Ns)) & (NFFT - 1)];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) ws[q] = tw[lane + 64 * q];
+
+  for (int64_t f = first; f < end; ++f) {
+    const int jlo = nlo, jhi = nhi, j0 = n0;
+    Cx v[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-      const int j = 2 * (lane + 64 * r);
-      v[r] = {sample(j), sample(j + 1)};
-    }
-  } else {
+      float e[2];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = {0.f, 0.f};
-  }
-  __syncthreads();  // twiddle table
+      for (int k = 0; k < 2; ++k) {
+        const int j = 2 * (lane + 64 * r) + k;
+        float y = __fsub_rn(raw[r][k + 1], __fmul_rn(preemph, raw[r][k]));
+        if (j == j0) y = raw[r][k + 1];  // sample 0 has no predecessor
+        e[k] = __fmul_rn(j >= jlo && j < jhi ? y : 0.f, win[r][k]);
+      }
+      v[r] = {e[0], e[1]};
+    }
+    if (f + 1 < end) load(f + 1);
 
-  // radix-4 Stockham passes, Ns = 1, 4, 16, 64: lane j combines in[j + 64 r] (twiddled by W_{4 Ns}^{r (j % Ns)}) and
-  // writes out[(j / Ns) 4 Ns + j % Ns + r Ns]
-  int cur = 0;
+    // radix-4 Stockham passes, Ns = 1, 4, 16, 64: lane j combines in[j + 64 r] (twiddled by W_{4 Ns}^{r (j % Ns)}) and
+    // writes out[(j / Ns) 4 Ns + j % Ns + r Ns]
+    int cur = 0;
 #pragma unroll
-  for (int Ns = 1; Ns < NZ; Ns *= 4) {
-    const int jm = lane % Ns;
-    if (Ns > 1) {
+    for (int Ns = 1; Ns < NZ; Ns *= 4) {
+      const int jm = lane % Ns;
+      if (Ns > 1) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) v[r] = buf[w][cur][lane + 64 * r];
+        for (int r = 0; r < 4; ++r) v[r] = buf[w][cur][lane + 64 * r];
 #pragma unroll
-      for (int r = 1; r < 4; ++r) v[r] = cmul(v[r], tw[(r * jm * (128 / Ns)) & (NFFT - 1)]);
-      cur ^= 1;
+        for (int r = 1; r < 4; ++r) v[r] = cmul(v[r], wp[Ns == 4 ? 0 : (Ns == 16 ? 1 : 2)][r - 1]);
+        cur ^= 1;
+      }
+      const Cx a0 = cadd(v[0], v[2]), a1 = csub(v[0], v[2]), a2 = cadd(v[1], v[3]), a3 = mul_mi(csub(v[1], v[3]));
+      const int o = (lane / Ns) * 4 * Ns + jm;
+      buf[w][cur][o] = cadd(a0, a2);
+      buf[w][cur][o + Ns] = cadd(a1, a3);
+      buf[w][cur][o + 2 * Ns] = csub(a0, a2);
+      buf[w][cur][o + 3 * Ns] = csub(a1, a3);
+      wave_lds_sync();
     }
-    const Cx a0 = cadd(v[0], v[2]), a1 = csub(v[0], v[2]), a2 = cadd(v[1], v[3]), a3 = mul_mi(csub(v[1], v[3]));
-    const int o = (lane / Ns) * 4 * Ns + jm;
-    buf[w][cur][o] = cadd(a0, a2);
-    buf[w][cur][o + Ns] = cadd(a1, a3);
-    buf[w][cur][o + 2 * Ns] = csub(a0, a2);
-    buf[w][cur][o + 3 * Ns] = csub(a1, a3);
-    __syncthreads();
-  }
-  // Z = buf[w][cur] in natural order. Bins of the real transform: X[k] = E[k] + W_512^k O[k] with
-  // E = (Z[k] + conj Z[256-k]) / 2, O = (Z[k] - conj Z[256-k]) / 2i; X[256] = E[0] - O[0]. Power as the extractor:
-  // |X| then squared.
-  const Cx* Z = buf[w][cur];
-  float* pw = power[w];
+    // Z = buf[w][cur] in natural order. Bins of the real transform: X[k] = E[k] + W_512^k O[k] with
+    // E = (Z[k] + conj Z[256-k]) / 2, O = (Z[k] - conj Z[256-k]) / 2i; X[256] = E[0] - O[0]. Power as the extractor:
+    // |X| then squared.
+    const Cx* Z = buf[w][cur];
+    float* pw = power[w];
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int k = lane + 64 * q;
-    const Cx zk = Z[k], zc0 = Z[(NZ - k) & (NZ - 1)];
-    const Cx zc = {zc0.re, -zc0.im};
-    const Cx e = {0.5f * (zk.re + zc.re), 0.5f * (zk.im + zc.im)};
-    const Cx d = csub(zk, zc);
-    const Cx o = {0.5f * d.im, -0.5f * d.re};  // d / 2i
-    const Cx X = cadd(e, cmul(tw[k], o));
-    const float a = __fsqrt_rn(__fadd_rn(__fmul_rn(X.re, X.re), __fmul_rn(X.im, X.im)));
-    pw[k] = __fmul_rn(a, a);
-    if (k == 0) {
-      const float x256 = e.re - o.re;  // E[0] and O[0] are real
-      const float a2 = __fsqrt_rn(__fmul_rn(x256, x256));
-      pw[NZ] = __fmul_rn(a2, a2);
+    for (int q = 0; q < 4; ++q) {
+      const int k = lane + 64 * q;
+      const Cx zk = Z[k], zc0 = Z[(NZ - k) & (NZ - 1)];
+      const Cx zc = {zc0.re, -zc0.im};
+      const Cx e = {0.5f * (zk.re + zc.re), 0.5f * (zk.im + zc.im)};
+      const Cx d = csub(zk, zc);
+      const Cx o = {0.5f * d.im, -0.5f * d.re};  // d / 2i
+      const Cx X = cadd(e, cmul(ws[q], o));
+      const float a = __fsqrt_rn(__fadd_rn(__fmul_rn(X.re, X.re), __fmul_rn(X.im, X.im)));
+      pw[k] = __fmul_rn(a, a);
+      if (k == 0) {
+        const float x256 = e.re - o.re;  // E[0] and O[0] are real
+        const float a2 = __fsqrt_rn(__fmul_rn(x256, x256));
+        pw[NZ] = __fmul_rn(a2, a2);
+      }
     }
-  }
-  __syncthreads();
-  // mel bands m = lane and lane + 64 (a narrow low band with a wide high one), fp32 over the band's nonzero bins in
-  // order; log(mel + 2^-24)
-  if (live) {
+    wave_lds_sync();
+    // mel bands m = lane and lane + 64 (a narrow low band with a wide high one), fp32 over the band's nonzero bins in
+    // order; log(mel + 2^-24)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int m = lane + 64 * h;
-      const float* wm = mel + (int64_t)m * BINS;
-      const int k0 = band[2 * m], k1 = band[2 * m + 1];
+      const int m = lane + 64 * h, near = min(k1[h], k0[h] + MTAPS);
       float acc = 0.f;
-      for (int k = k0; k < k1; ++k) acc = __builtin_fmaf(wm[k], pw[k], acc);
+      for (int k = k0[h]; k < near; ++k) acc = __builtin_fmaf(mw[k - k0[h]][m], pw[k], acc);
+      for (int k = near; k < k1[h]; ++k) acc = __builtin_fmaf(mel[(int64_t)m * BINS + k], pw[k], acc);
       logmel[f * MELS + m] = logf(__fadd_rn(acc, 5.9604644775390625e-8f));
     }
+    wave_lds_sync();  // the powers are read before the next frame's
   }
 }
 
-// per piece and mel band: mean and unbiased variance over the piece's valid frames (fp64 sums, 16 frame groups added
-// in a fixed order), then (v - mean) / (std + 1e-5) as bf16 into out (pieces, T, 128) at the piece's first frames.
-// Workgroup (piece, 16 bands): thread (g, m) = frames g, g + 16, ... of band 16 blockIdx.y + m.
-constexpr int NG = 16, MB = 16;
-__global__ void __launch_bounds__(NG* MB) normalize_kernel(const float* __restrict__ logmel,
-                                                           const int64_t* __restrict__ frame_start, int64_t T,
-                                                           uint16_t* __restrict__ out) {
-  __shared__ double part[NG][MB];
-  const int p = blockIdx.x, m = threadIdx.x % MB, g = threadIdx.x / MB, band = blockIdx.y * MB + m;
+// per piece and mel band: mean and unbiased variance over the piece's valid frames (fp64 sums in a fixed order), then
+// (v - mean) / (std + 1e-5) as bf16 into out (pieces, T, 128) at the piece's first frames.
+// Bound by memory latency: the bytes are few (6.6 MB read, 3.3 MB written for eight pieces of 2 to 30 s) and a piece's
+// two sums come one after the other. A workgroup takes 8 bands of a piece: thread (f, q) holds bands 4 q .. 4 q + 3 of
+// frames f, f + 512, ... in registers, so the values are read once for both sums and the output, 512 frames in flight
+// (only past NKEEP * 512 frames, 30.7 s, are they read again). 16 bands of 16 frames in flight, read three times over,
+// took 101 us there, this 15 us. The 16 workgroups of a piece run on one XCD (contiguous items of the remapped
+// index), whose L2 then merges their 16-byte parts of each output row.
+// four floats / four bf16 values, read or written whole at their own alignment
+typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t b4_any __attribute__((ext_vector_type(2), aligned(2)));
+constexpr int NB = 8, NQ = NB / 4, NTHR = 1024, NFR = NTHR / NQ, NKEEP = 6;
+__global__ void __launch_bounds__(NTHR) normalize_kernel(const float* __restrict__ logmel,
+                                                         const int64_t* __restrict__ frame_start, int64_t T,
+                                                         uint16_t* __restrict__ out) {
+  __shared__ double part[NTHR / 64][NB];
+  const int total = (int)gridDim.x, xcd = (int)blockIdx.x % 8;  // workgroup b runs on XCD b % 8
+  const int item = xcd * (total / 8) + min(xcd, total % 8) + (int)blockIdx.x / 8;
+  const int p = item / (MELS / NB), b0 = item % (MELS / NB) * NB;
+  const int tid = threadIdx.x, q = tid % NQ, f = tid / NQ, wave = tid >> 6;
   const int64_t f0 = frame_start[p], nv = frame_start[p + 1] - f0;
   if (nv == 0) return;
-  const float* v = logmel + f0 * MELS + band;
-  uint16_t* o = out + (int64_t)p * T * MELS + band;
-  auto total = [&](double s) {
-    part[g][m] = s;
-    __syncthreads();
-    double t = 0.0;
+  const float* v = logmel + f0 * MELS + b0 + 4 * q;
+  uint16_t* o = out + (int64_t)p * T * MELS + b0 + 4 * q;
+  v4f keep[NKEEP];
 #pragma unroll
-    for (int k = 0; k < NG; ++k) t += part[k][m];
-    __syncthreads();
-    return t;
-  };
-  double s = 0.0;
-  for (int64_t t = g; t < nv; t += NG) s += v[t * MELS];
-  const float mean = (float)(total(s) / (double)nv);
-  double q = 0.0;
-  for (int64_t t = g; t < nv; t += NG) {
-    const double d = (double)v[t * MELS] - (double)mean;
-    q += d * d;
+  for (int i = 0; i < NKEEP; ++i) {
+    const int64_t t = f + (int64_t)i * NFR;
+    keep[i] = t < nv ? (v4f) * reinterpret_cast<const f4_any*>(v + t * MELS) : v4f{0.f, 0.f, 0.f, 0.f};
   }
-  const float den = __fadd_rn((float)sqrt(total(q) / (double)(nv - 1)), 1e-5f);
-  for (int64_t t = g; t < nv; t += NG) o[t * MELS] = f2bf(__fdiv_rn(__fsub_rn(v[t * MELS], mean), den));
+  // the workgroup's sum of each band, in every thread of that band: over the wave's lanes of equal q, then its waves
+  auto total_of = [&](double (&s)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+#pragma unroll
+      for (int d = NQ; d < 64; d <<= 1) s[k] += __shfl_xor(s[k], d, 64);
+    }
+    __syncthreads();  // the last sums are read
+    if ((tid & 63) < NQ)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) part[wave][4 * q + k] = s[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      double t = 0.0;
+#pragma unroll
+      for (int w = 0; w < NTHR / 64; ++w) t += part[w][4 * q + k];
+      s[k] = t;
+    }
+  };
+  auto each = [&](auto fn) {  // this thread's frames, the kept ones first
+#pragma unroll
+    for (int i = 0; i < NKEEP; ++i) {
+      const int64_t t = f + (int64_t)i * NFR;
+      if (t < nv) fn(t, keep[i]);
+    }
+    for (int64_t t = f + (int64_t)NKEEP * NFR; t < nv; t += NFR)
+      fn(t, (v4f) * reinterpret_cast<const f4_any*>(v + t * MELS));
+  };
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  each([&](int64_t, const v4f& x) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s[k] += x[k];
+  });
+  total_of(s);
+  float mean[4], den[4];
+  double m2[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int k = 0; k < 4; ++k) mean[k] = (float)(s[k] / (double)nv);
+  each([&](int64_t, const v4f& x) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const double d = (double)x[k] - (double)mean[k];
+      m2[k] += d * d;
+    }
+  });
+  total_of(m2);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) den[k] = __fadd_rn((float)sqrt(m2[k] / (double)(nv - 1)), 1e-5f);
+  each([&](int64_t t, const v4f& x) {
+    float y[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) y[k] = __fdiv_rn(__fsub_rn(x[k], mean[k]), den[k]);
+    *reinterpret_cast<b4_any*>(o + t * MELS) = b4_any{pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3])};
+  });
 }
 
 // ---- subsampling convolutions ------------------------------------------------------------------------------------
@@ -332,11 +440,14 @@ extern "C" int cohere_logmel_features(const float* x, const int64_t* meta, int64
   if (total_frames == 0 || pieces == 0) return 0;
   COHERE_REQUIRE(x && meta && window && mel && band && out && work, "logmel_features: null pointer");
   const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int64_t blocks = (total_frames + FPW - 1) / FPW;
-  COHERE_REQUIRE(blocks < (1LL << 31), "logmel_features: too many frames");
-  logmel_kernel<<<(unsigned)blocks, FPW * 64, 0, s>>>(x, meta, (int)pieces, total_frames, window, mel, band, preemph,
-                                                       work);
-  normalize_kernel<<<dim3((unsigned)pieces, MELS / MB), NG * MB, 0, s>>>(work, meta + 2 * pieces, T, out);
+  // frames per wave: as many as keep four workgroups for each of 256 CUs (a workgroup's tables cost about as much as
+  // three frames)
+  const int64_t per_wave = std::min<int64_t>(8, std::max<int64_t>(1, total_frames / (FPW * 1024)));
+  const int64_t blocks = (total_frames + FPW * per_wave - 1) / (FPW * per_wave);
+  COHERE_REQUIRE(blocks < (1LL << 31) && pieces * (MELS / NB) < (1LL << 31), "logmel_features: too many frames");
+  logmel_kernel<<<(unsigned)blocks, FPW * 64, 0, s>>>(x, meta, (int)pieces, total_frames, (int)per_wave, window, mel,
+                                                       band, preemph, work);
+  normalize_kernel<<<(unsigned)(pieces * (MELS / NB)), NTHR, 0, s>>>(work, meta + 2 * pieces, T, out);
   return cohere::check_launch("logmel_features");
 }
 
