@@ -21,7 +21,7 @@ OUT_DIR = os.path.join(PKG, "lib")
 LIB = os.path.join(OUT_DIR, "libcohere_hip.so")
 OBJ_DIR = os.path.join(ROOT, "_build")
 
-SOURCES = ["capi.cpp", "gemm_q8.hip", "gemm_q8_dense.hip", "gemm_q8_sparse.hip", "dec_w8.hip", "quant.hip",
+SOURCES = ["capi.cpp", "gemm_q8.hip", "gemm_q8_dense.hip", "gemm_q8_sparse.hip", "gemm_q8_rows.hip", "dec_w8.hip", "quant.hip",
            "encoder_ops.hip", "encoder_loop.cpp", "encoder_noalloc.hip", "decoder_ops.hip", "gemm_bf16.hip", "frontend.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"

@@ -12,6 +12,8 @@
 //   OUT:  x = LN_out(x) and, fused, hq = LN_ff1 of the next layer (the last layer: x = LN_out(x) in bf16)
 #include "cohere_hip.h"
 #include "common.h"
+#include "gemm_q8.h"
+#include "gemm_q8_rows.h"
 
 #include <algorithm>
 #include <string>
@@ -180,6 +182,128 @@ int encoder_layers_bf16(uint16_t* x, int64_t rows, const void* const* fields, in
   return 0;
 }
 
+// ---- few rows ----------------------------------------------------------------------------------------------------
+
+bool al16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
+
+// Whether the few-row launch sequence takes this call: few rows, 256-column feed-forward groups, and every argument
+// one that the general sequence would accept (it words the refusals).
+bool few_rows(const uint16_t* x, int64_t rows, const void* const* fields, int64_t n_layers, int64_t group,
+              int64_t c_i8, int64_t c_grp, int64_t c_ff1, int64_t c_pw1, int64_t c_o, int64_t c_sp) {
+  if (rows > cohere_rows_gemm::ROWS_MAX || group != cohere_rows_gemm::UNIT || !al16(x)) return false;
+  for (int64_t c : {c_i8, c_grp, c_pw1, c_o})
+    if (cohere_gemm::ref_config_group((int)c) == -2) return false;
+  if (c_sp < -1 || c_sp > 4 || cohere_gemm::ref_config_group((int)c_ff1) != group) return false;
+  static const int lns[] = {LN_FF1_W, LN_FF1_B, LN_ATT_W, LN_ATT_B, LN_CONV_W, LN_CONV_B, LN_FF2_W, LN_FF2_B};
+  static const int mats[] = {Q_FF1_W1, Q_FF1_W2, Q_FF2_W1, Q_FF2_W2, Q_QKV_W, Q_PW1_W, Q_O_W, Q_PW2_W, SP_FF1_W,
+                             SP_FF1_E, SP_FF2_W, SP_FF2_E, SP_FF1_W1, SP_FF1_E1, SP_FF2_W1, SP_FF2_E1, Q_FF1_S1,
+                             Q_FF1_S2, Q_FF2_S1, Q_FF2_S2, Q_QKV_S, Q_PW1_S, Q_O_S, Q_PW2_S};
+  static const int biases[] = {FF1_B1, FF1_B2, FF2_B1, FF2_B2, BQKV, BO, BPW1, BPW2};
+  for (int64_t l = 0; l < n_layers; ++l) {
+    const void* const* ly = fields + l * N_FIELDS;
+    for (int f : lns)
+      if (!al16(ly[f])) return false;
+    for (int f : mats)
+      if (!al16(ly[f])) return false;
+    for (int f : biases)
+      if (reinterpret_cast<uintptr_t>(ly[f]) & 7) return false;
+  }
+  return true;
+}
+
+// The int8 layers over few rows, with the general sequence's bits: the attention's output is quantized by its projection
+// (the few-row GEMM, gemm_q8_rows.hip), and the feed-forwards' hidden rows stay bf16 (over the QKV and attention
+// buffers, idle then) and are quantized per 256 columns by the second linear, so that the first needs no 256-column
+// workgroups. One block of 26 rows 140 -> 83 us, 64 rows 146 -> 90, 96 rows 123 -> 92 (W2 2:4).
+int encoder_layers_few(uint16_t* x, int64_t rows, const void* const* fields, int64_t n_layers, const double* eps,
+                       const int32_t* tiles, int64_t n_tiles, const int32_t* lo, const int32_t* hi, int64_t rel_off,
+                       int64_t max_len, int64_t rel_rows, double scale, int32_t heads, int32_t head_dim,
+                       int64_t c_i8, int64_t c_pw1, int64_t c_o, const Workspace& ws, void* stream) {
+  namespace R = cohere_rows_gemm;
+  const hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  auto ep = [&](int64_t i, int e) { return (float)eps[i * N_EPS + e]; };
+  int64_t i = 0;
+  auto fail = [&](const char* what) {
+    cohere::set_error("encoder_layers: layer " + std::to_string(i) + ", " + what + ": " + cohere_last_error());
+    return 1;
+  };
+#define RUN(call, what) \
+  if ((call) != 0) return fail(what)
+  uint16_t* hidden = ws.qkv;  // (rows, 5120): the QKV and attention buffers are 3840 + 1280 columns
+  auto normalise = [&](const void* const* ly, int w, int b, float e) {  // LayerNorm of x into hq, hs
+    return cohere_layernorm_q8(x, DM, fld<uint16_t>(ly, w), fld<uint16_t>(ly, b), e, nullptr, nullptr, 0.f, ws.hq, DM,
+                               ws.hs, rows, DM, stream);
+  };
+  auto gemm = [&](const void* const* ly, int w, int s, int b, uint16_t* y, int64_t n, int epi, int64_t cfg) {  // of hq
+    const bool onto = epi == COHERE_EPI_RESID;
+    const int64_t ld = epi == COHERE_EPI_GLU ? n / 2 : n;
+    return cohere_gemm_i8(ws.hq, DM, ws.hs, 1, DM, fld<int8_t>(ly, w), fld<float>(ly, s), fld<uint16_t>(ly, b), y, ld,
+                          epi, onto ? y : nullptr, ld, 1.f, nullptr, 0, rows, n, DM, (int32_t)cfg, stream);
+  };
+  // hidden = bf16(silu(hq W1 + b))
+  auto w1 = [&](const void* const* ly, int w, int s, int b, int spw, int spe) {
+    cohere_gemm::GemmArgs p{};
+    const bool sparse = ly[spw] != nullptr;
+    p.X = ws.hq; p.ldx = DM; p.sx = ws.hs; p.ldsx = 1;
+    p.W = fld<int8_t>(ly, sparse ? spw : w); p.E = fld<int32_t>(ly, spe); p.tiled = sparse && !p.E;
+    if (p.tiled) p.E = reinterpret_cast<const int32_t*>(p.W);
+    p.sw = fld<float>(ly, s); p.bias = fld<uint16_t>(ly, b); p.C = hidden; p.ldc = DFF; p.alpha = 1.f;
+    p.M = (int)rows; p.N = (int)DFF; p.K = (int)DM; p.group = (int)DM; p.qgroup = 256; p.epi = cohere_gemm::EPI_SILU;
+    if (sparse) cohere_gemm::launch_silu_few<true>(p, st);
+    else cohere_gemm::launch_silu_few<false>(p, st);
+    return cohere::check_launch("feed-forward W1");
+  };
+  // x = x + alpha (bf16 rows, quantized W + b)
+  auto onto_x = [&](const uint16_t* rows_bf, int64_t k, R::XMode xm, float alpha, const void* const* ly, int w, int s,
+                    int b, int spw, int spe) {
+    R::Args a{};
+    const bool sparse = spw >= 0 && ly[spw];
+    a.X = rows_bf; a.ldx = k; a.W = fld<int8_t>(ly, sparse ? spw : w); a.E = sparse ? fld<int32_t>(ly, spe) : nullptr;
+    a.tiled = sparse && !a.E; a.sw = fld<float>(ly, s); a.bias = fld<uint16_t>(ly, b);
+    a.Y = x; a.ldy = DM; a.R = x; a.ldr = DM; a.alpha = alpha; a.M = (int)rows; a.N = (int)DM; a.K = (int)k;
+    if (!R::launch(xm, sparse, COHERE_EPI_RESID, a, st)) {
+      cohere::set_error("no few-row kernel");
+      return 1;
+    }
+    return cohere::check_launch("few-row linear");
+  };
+  RUN(normalise(fields, LN_FF1_W, LN_FF1_B, ep(0, EPS_FF1)), "first LayerNorm");
+  for (i = 0; i < n_layers; ++i) {
+    const void* const* ly = fields + i * N_FIELDS;
+    RUN(w1(ly, Q_FF1_W1, Q_FF1_S1, FF1_B1, SP_FF1_W1, SP_FF1_E1), "feed-forward 1 W1");
+    RUN(onto_x(hidden, DFF, R::X_BFG, 0.5f, ly, Q_FF1_W2, Q_FF1_S2, FF1_B2, SP_FF1_W, SP_FF1_E), "feed-forward 1 W2");
+    RUN(normalise(ly, LN_ATT_W, LN_ATT_B, ep(i, EPS_ATT)), "attention LayerNorm");
+    RUN(gemm(ly, Q_QKV_W, Q_QKV_S, BQKV, ws.qkv, DQKV, COHERE_EPI_BIAS, c_i8), "QKV");
+    RUN(cohere_relpos_attention(ws.qkv, fld<uint16_t>(ly, RK), rel_rows, fld<uint16_t>(ly, BU),
+                                fld<uint16_t>(ly, BV), tiles, n_tiles, heads, head_dim, rel_off, max_len,
+                                (float)scale, ws.a, stream),
+        "attention");
+    RUN(onto_x(ws.a, DM, R::X_BF, 1.f, ly, Q_O_W, Q_O_S, BO, -1, -1), "attention output projection");
+    RUN(normalise(ly, LN_CONV_W, LN_CONV_B, ep(i, EPS_CONV)), "convolution LayerNorm");
+    RUN(gemm(ly, Q_PW1_W, Q_PW1_S, BPW1, ws.a, 2 * DM, COHERE_EPI_GLU, c_pw1), "pointwise conv 1 (GLU)");
+    RUN(cohere_dwconv_bn_silu_q8(ws.a, fld<float>(ly, WDW), fld<float>(ly, BDW), fld<float>(ly, BN_SCALE),
+                                 fld<float>(ly, BN_SHIFT), lo, hi, ws.hq, ws.hs, rows, DM, 9, stream),
+        "depthwise conv");
+    RUN(gemm(ly, Q_PW2_W, Q_PW2_S, BPW2, x, DM, COHERE_EPI_RESID, c_o), "pointwise conv 2");
+    RUN(normalise(ly, LN_FF2_W, LN_FF2_B, ep(i, EPS_FF2)), "feed-forward 2 LayerNorm");
+    RUN(w1(ly, Q_FF2_W1, Q_FF2_S1, FF2_B1, SP_FF2_W1, SP_FF2_E1), "feed-forward 2 W1");
+    RUN(onto_x(hidden, DFF, R::X_BFG, 0.5f, ly, Q_FF2_W2, Q_FF2_S2, FF2_B2, SP_FF2_W, SP_FF2_E), "feed-forward 2 W2");
+    if (i + 1 < n_layers) {
+      const void* const* nx = ly + N_FIELDS;
+      RUN(cohere_layernorm_q8(x, DM, fld<uint16_t>(ly, LN_OUT_W), fld<uint16_t>(ly, LN_OUT_B), ep(i, EPS_OUT),
+                              fld<uint16_t>(nx, LN_FF1_W), fld<uint16_t>(nx, LN_FF1_B), ep(i + 1, EPS_FF1), ws.hq, DM,
+                              ws.hs, rows, DM, stream),
+          "output LayerNorm");
+    } else {
+      RUN(cohere_layernorm(x, DM, fld<uint16_t>(ly, LN_OUT_W), fld<uint16_t>(ly, LN_OUT_B), ep(i, EPS_OUT), nullptr,
+                           nullptr, 0.f, x, DM, rows, DM, stream),
+          "output LayerNorm");
+    }
+  }
+#undef RUN
+  return 0;
+}
+
 }  // namespace
 
 extern "C" int cohere_encoder_layers(uint16_t* x, int64_t rows, const void* const* fields, int64_t n_layers,
@@ -221,6 +345,9 @@ extern "C" int cohere_encoder_layers(uint16_t* x, int64_t rows, const void* cons
                        ": a feed-forward linear has neither dense nor 2:4 weights");
   }
 
+  if (few_rows(x, rows, fields, n_layers, group, c_i8, c_grp, c_ff1, c_pw1, c_o, c_sp))
+    return encoder_layers_few(x, rows, fields, n_layers, eps, tiles, n_tiles, lo, hi, rel_off, max_len, rel_rows, scale,
+                              heads, head_dim, c_i8, c_pw1, c_o, ws, stream);
   const int64_t ts_ld = DFF / group;
   auto ep = [&](int64_t i, int e) { return (float)eps[i * N_EPS + e]; };
   auto fail = [&](int64_t i, const char* what) {

@@ -41,7 +41,8 @@
 
 namespace cohere_gemm {
 
-// the reference's epilogue ids (kernels/cuda_ext.py:28); SILU, RELU and CONV_RELU are bf16-operand only, I32 is ours
+// the reference's epilogue ids (kernels/cuda_ext.py:28); RELU and CONV_RELU are bf16-operand only (SILU too through the
+// C ABI; the few-row layers use it on int8 operands), I32 is ours
 enum { EPI_BIAS = 0, EPI_SILU = 1, EPI_RELU = 2, EPI_RESID = 3, EPI_GLU = 4, EPI_SILU_Q8 = 5, EPI_CONV_RELU = 6,
        EPI_I32 = 7 };
 
@@ -167,7 +168,7 @@ template <int BM, int BN, int WM, int WN, int ST, int MS, int EPI, bool GROUPED,
           bool BF = false>
 __global__ void __launch_bounds__(WM* WN * 64) gemm_q8_kernel(const GemmArgs p) {
   static_assert(!BF || (!SPARSE && !GROUPED && EPI != EPI_SILU_Q8 && EPI != EPI_I32), "bf16 operands");
-  static_assert(BF || (EPI != EPI_SILU && EPI != EPI_RELU && EPI != EPI_CONV_RELU), "bf16-only epilogue");
+  static_assert(BF || (EPI != EPI_RELU && EPI != EPI_CONV_RELU), "bf16-only epilogue");
   using T = Tile<BM, BN, WM, WN, ST, MS, GROUPED, SPARSE>;
   constexpr int NW = T::NW, NT = T::NT, TM = T::TM, TN = T::TN, MI = T::MI, NI = T::NI, LPS = T::LPS;
   constexpr int KSTEP = T::KSTEP, SPS = T::SPS, RPL = T::RPL;
@@ -833,6 +834,15 @@ bool launch_tiles(int tile, const GemmArgs& p, hipStream_t s) {
 // instantiated in gemm_q8_dense.hip / gemm_q8_sparse.hip
 template <bool SPARSE>
 bool launch_gemm(int tile, int epi, bool grouped, const GemmArgs& p, hipStream_t s);
+
+// y = bf16(silu(bf16(dequant(x W^T) + bias))) of few int8 rows: SILU_Q8's values before their quantization, on the
+// 64 x 64 tile, which gives the 5120-wide feed-forward linear 80 workgroups per 64 rows (SILU_Q8 needs a whole
+// 256-column group per workgroup: 20). Arguments as the C entry points check them; N % 64 == 0.
+template <bool SPARSE>
+void launch_silu_few(const GemmArgs& p, hipStream_t s);
+
+// the SILU_Q8 output group of an int8 config id, -2 for an unknown id
+int ref_config_group(int cfg);
 
 // bf16 operands (instantiated in gemm_bf16.hip): the tiles with a bf16 instantiation, and the launch
 constexpr bool bf16_tile(int tile) { return tile == 0 || tile == 1 || tile == 3 || tile == 6 || tile == 7 || tile == 9; }

@@ -2,6 +2,7 @@
 // choice of gfx950 tile, and dispatch to the kernel instantiations (gemm_q8.h, gemm_q8_dense.hip, gemm_q8_sparse.hip).
 #include "cohere_hip.h"
 #include "gemm_q8.h"
+#include "gemm_q8_rows.h"
 
 #include <cstring>
 #include <string>
@@ -73,6 +74,20 @@ int ref_cfg_group(int cfg) {
   }
 }
 
+// Few rows go to the few-row kernel where it is the faster one (the same bits; a forced tile keeps the tile GEMM)
+bool rows_gemm(const GemmArgs& p, bool sparse, bool grouped, hipStream_t s) {
+  namespace R = cohere_rows_gemm;
+  if (g_tile_override >= 0 || !R::better_than_tiles(p.M, p.N, p.K)) return false;
+  if (p.epi != EPI_BIAS && p.epi != EPI_RESID && p.epi != EPI_GLU) return false;
+  if (grouped && p.group != R::UNIT) return false;
+  R::Args a{};
+  a.X = p.X; a.sx = p.sx; a.W = p.W; a.E = p.E; a.sw = p.sw; a.bias = p.bias;
+  a.Y = static_cast<uint16_t*>(p.C); a.R = p.R;
+  a.ldx = p.ldx; a.ldsx = p.ldsx; a.ldy = p.ldc; a.ldr = p.ldr;
+  a.M = p.M; a.N = p.N; a.K = p.K; a.tiled = p.tiled; a.alpha = p.alpha;
+  return R::launch(grouped ? R::X_Q8G : R::X_Q8, sparse, p.epi, a, s);
+}
+
 bool aligned16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
 
 template <bool SPARSE>
@@ -104,6 +119,7 @@ int gemm_entry(GemmArgs& p, int64_t group, int64_t lda_k_req, hipStream_t s, con
   COHERE_REQUIRE(p.epi != EPI_RESID || (aligned16(p.R) && p.ldr % 8 == 0), nm + ": residual rows must be aligned");
   if (p.M == 0) return 0;
   p.group = (int)group;
+  if (rows_gemm(p, SPARSE, grouped, s)) return cohere::check_launch(name);
   const int tile = choose_tile(p, grouped);
   COHERE_REQUIRE(tile >= 0, nm + ": no gfx950 tile fits N=" + std::to_string(p.N));
   if (!launch_gemm<SPARSE>(tile, p.epi, grouped, p, s)) {
@@ -114,6 +130,8 @@ int gemm_entry(GemmArgs& p, int64_t group, int64_t lda_k_req, hipStream_t s, con
 }
 
 }  // namespace
+
+int cohere_gemm::ref_config_group(int cfg) { return ref_cfg_group(cfg); }
 
 extern "C" int cohere_set_gemm_tile(int32_t tile) {
   if (tile == -2 || tile == -3) {  // the XCD split off / on

@@ -24,4 +24,9 @@ bool launch_gemm<false>(int tile, int epi, bool grouped, const GemmArgs& p, hipS
   }
 }
 
+template <>
+void launch_silu_few<false>(const GemmArgs& p, hipStream_t s) {
+  launch_tile<64, 64, 2, 2, 4, 16, EPI_SILU, false, false>(p, s);
+}
+
 }  // namespace cohere_gemm

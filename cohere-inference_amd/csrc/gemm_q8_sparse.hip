@@ -24,4 +24,9 @@ bool launch_gemm<true>(int tile, int epi, bool grouped, const GemmArgs& p, hipSt
   }
 }
 
+template <>
+void launch_silu_few<true>(const GemmArgs& p, hipStream_t s) {
+  launch_tile<64, 64, 2, 2, 4, 16, EPI_SILU, false, true>(p, s);
+}
+
 }  // namespace cohere_gemm

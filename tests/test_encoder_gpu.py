@@ -228,3 +228,17 @@ def test_encoder_layers_bf16(gpu):
     print(f"bf16 layers: kernels vs checker rms {rms_gpu:.2e} max {max_gpu:.2e}; perturbed checker rms "
           f"{rms_noise:.2e} max {max_noise:.2e}")
     assert rms_gpu < rms_noise and max_gpu <= 2 * max_noise
+
+
+@pytest.mark.parametrize("lengths,sparse,sparse_w1", [([96], True, True), ([1], False, False), ([26, 17], True, False),
+                                                      ([33], False, True), ([16], True, False)])
+def test_encoder_layers_few_rows(gpu, lengths, sparse, sparse_w1):
+    """Calls of at most 96 rows run the few-row launches. A piece is independent of the pieces beside it and both
+    sequences do the same arithmetic, so the same rows inside a call of more rows give the same bits."""
+    layers = product_layers(gpu, 1, 41, sparse, sparse_w1)
+    g = torch.Generator().manual_seed(sum(lengths))
+    x = torch.randn(sum(lengths) + 100, 1280, generator=g).to(torch.bfloat16).to(gpu)
+    print(f"few rows {lengths}", flush=True)
+    few = layers(x[:sum(lengths)].clone(), lengths)
+    many = layers(x.clone(), [*lengths, 100])[:sum(lengths)]
+    assert np.array_equal(_bits(few), _bits(many))

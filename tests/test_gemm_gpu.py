@@ -367,3 +367,46 @@ def test_empty_rows_noop(ext):
     out = torch.empty(0, 64, dtype=torch.bfloat16, device="cuda")
     ext.gemm_i8(xq, xs, 128, wq, torch.ones(64, device="cuda"), None, out, EPI_BIAS, None, 1.0, None, 0)
     torch.cuda.synchronize()
+
+
+# ---- few rows: the kernel of csrc/gemm_q8_rows.hip ----------------------------------------------------------------------
+
+@pytest.mark.parametrize("M", [1, 15, 17, 96])
+@pytest.mark.parametrize("N,K,group", [(64, 256, 256), (512, 1280, 1280), (1280, 5120, 256), (960, 2816, 2816)])
+def test_few_rows_same_bits_as_tiles(ext, M, N, K, group):
+    """At most 96 rows take the few-row kernel (1 and 2 strips a workgroup, units that divide evenly over its waves and
+    not): dense, row-major 2:4 and stage-tiled 2:4, BIAS / RESID / GLU, per-row and grouped scales, with and without
+    bias, equal the tile GEMM (a forced tile) bit for bit."""
+    from kernels.cuda_ext import EPI_BIAS, EPI_GLU, EPI_RESID
+    from kernels.fast_encoder import quantize_rows
+    from kernels.sparse import compress_24, pack_24_tiled, prune_24_magnitude
+
+    print(f"few rows M={M} N={N} K={K} group={group}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    xq = torch.randint(-127, 128, (M, K), generator=g, dtype=torch.int8).cuda()
+    xs = (torch.rand(M, K // group, generator=g) * 0.02 + 1e-3).cuda()
+    w = (torch.randn(N, K, generator=g) * 0.02).to(torch.bfloat16)
+    b = (torch.randn(N, generator=g) * 0.01).to(torch.bfloat16).cuda()
+    r = torch.randn(M, N, generator=g).to(torch.bfloat16).cuda()
+    wq, ws = quantize_rows(prune_24_magnitude(w))
+    wc, e = compress_24(wq)
+    wq, ws, wc, e, wt = wq.cuda(), ws.cuda(), wc.cuda(), e.cuda(), pack_24_tiled(wc, e).cuda()
+    for epi in ((EPI_RESID,) if group < K else (EPI_BIAS, EPI_RESID, EPI_GLU)):
+        for bias in (b, None):
+            outs = []
+            for tile in (7, -1):
+                ext.set_gemm_tile(tile)
+                for form in ("dense", "rows", "tiled"):
+                    out = r.clone() if epi == EPI_RESID else torch.empty(M, N // 2 if epi == EPI_GLU else N,
+                                                                        dtype=torch.bfloat16, device="cuda")
+                    res = out if epi == EPI_RESID else None
+                    if form == "dense":
+                        ext.gemm_i8(xq, xs, group, wq, ws, bias, out, epi, res, 0.5, None, 0)
+                    elif form == "rows":
+                        ext.gemm_sp_epi(xq, xs, group, wc, e, ws, bias, out, epi, res, 0.5, None, 0)
+                    else:
+                        ext.gemm_sp_tiled(xq, xs, group, wt, ws, bias, out, epi, res, 0.5, None, 0)
+                    outs.append(bf16_bits(out))
+            ext.set_gemm_tile(-1)
+            for o in outs[1:]:
+                assert np.array_equal(o, outs[0]), (epi, bias is None)
