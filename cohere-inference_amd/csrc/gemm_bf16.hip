@@ -10,10 +10,12 @@ template <int EPI>
 bool tiles_bf16(int tile, const GemmArgs& p, hipStream_t s) {
   switch (tile) {
     case 0: launch_tile<128, 128, 2, 2, 4, 16, EPI, false, false, true>(p, s); return true;
-    case 1: launch_tile<128, 256, 2, 2, 3, 16, EPI, false, false, true>(p, s); return true;
     case 3: launch_tile<64, 128, 2, 2, 4, 16, EPI, false, false, true>(p, s); return true;
     case 6: launch_tile<256, 256, 2, 4, 2, 16, EPI, false, false, true>(p, s); return true;
     case 7: launch_tile<64, 64, 2, 2, 4, 16, EPI, false, false, true>(p, s); return true;
+    case 8: launch_tile<256, 128, 4, 2, 3, 16, EPI, false, false, true>(p, s); return true;
+    case 15: launch_tile<256, 256, 4, 4, 2, 16, EPI, false, false, true>(p, s); return true;
+    case 17: launch_tile<128, 128, 2, 4, 4, 16, EPI, false, false, true>(p, s); return true;
     case 9: launch_tile<128, 256, 2, 4, 3, 16, EPI, false, false, true>(p, s); return true;
     default: return false;
   }

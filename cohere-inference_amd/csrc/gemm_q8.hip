@@ -13,8 +13,6 @@ using namespace cohere_gemm;
 
 int g_tile_override = -1;
 
-// gfx950 tile choice: the largest tile that still gives (nearly) every CU a workgroup; with fewer tiles than CUs,
-// the shape with the most workgroups. SILU_Q8 needs whole scale groups inside a tile.
 int num_cus() {
   static int n = [] {
     int dev = 0, v = 0;
@@ -26,6 +24,29 @@ int num_cus() {
   return n;
 }
 
+// The time of a round of workgroups, one per CU (64x64 tiles: two, the second costing a quarter more), on each tile, in
+// microseconds: c per 128-byte K stage, f for the launch, the first stage and the epilogue, q8 for SILU_Q8's. Fitted
+// to graph replays of the encoder's linears at 376, 1892, 3000 and 8416 rows (K 1280 and 5120) and the bf16 stem, cross-
+// attention and layer shapes; the model is within 10 % of most of them. Against the largest tile that gives 64 % of
+// the CUs a workgroup (the former rule): bf16 1892 x 1280 x 5120 62.2 -> 39.1 us, 1892 x 5120 x 1280 SILU 48.3 -> 39.7,
+// 1892 x 1280 x 1280 21.4 -> 13.9, 3000 x 1024 x 1280 15.0 -> 12.6; int8 3000 x 1280 x 1280 12.2 -> 9.5, grouped 1892 x
+// 1280 x 5120 42.7 -> 28.3.
+struct TileCost {
+  int id;
+  int per_cu;
+  double c, f, q8;
+};
+constexpr TileCost DENSE_COST[] = {{6, 1, 1.28, 10.9, 8.0}, {15, 1, 1.335, 10.0, 6.2}, {8, 1, .695, 7.5, 3.0},
+                                   {9, 1, .69, 6.6, 3.0},   {17, 1, .42, 4.5, 2.0},    {4, 1, .6, 4.0, 3.3},
+                                   {3, 1, .353, 3.3, 2.0},  {5, 1, .27, 3.1, 2.0},     {7, 2, .265, 3.0, 2.0}};
+// 2:4 weights; 10 reads stage-tiled records (row-major ones take 15)
+constexpr TileCost SPARSE_COST[] = {{10, 1, 1.03, 11.2, 7.0}, {15, 1, 1.25, 11.0, 7.0}, {8, 1, .58, 6.2, 3.5},
+                                    {9, 1, .52, 6.7, 3.5},    {17, 1, .47, 2.6, 2.0},   {0, 1, .437, 3.6, 2.0}, {4, 1, .447, 3.4, 4.1},
+                                    {3, 1, .35, 3.3, 2.0},    {5, 1, .27, 3.1, 2.0},    {7, 2, .25, 3.0, 2.0}};
+// grouped scales (each group's fold is most of a stage); the larger 8-wave tiles spill
+constexpr TileCost GROUPED_COST[] = {{17, 1, .62, 3.6, 2.0}, {4, 1, .75, 3.5, 3.3},  {3, 1, .47, 3.4, 2.0},
+                                     {5, 1, .35, 3.1, 2.0},  {7, 2, .34, 3.0, 2.0}};
+
 int choose_tile(const GemmArgs& p, bool grouped, bool bf = false) {
   auto fits = [&](int id) {
     const TileInfo& t = TILES[id];
@@ -36,29 +57,25 @@ int choose_tile(const GemmArgs& p, bool grouped, bool bf = false) {
     return true;
   };
   if (g_tile_override >= 0 && g_tile_override < N_TILES && fits(g_tile_override)) return g_tile_override;
-  auto tiles_of = [&](int id) { return (int64_t)((p.M + TILES[id].bm - 1) / TILES[id].bm) * (p.N / TILES[id].bn); };
-  // largest first; the first shape that gives about two thirds of the CUs a workgroup wins (measured on the encoder
-  // block's GEMMs at 1504-3000 rows: a large tile on 64 % of the CUs beats a smaller one on all of them). The 128x128
-  // tile on 32x32 instructions (12) precedes its 16x16 twin (0). Grouped scales skip 12 and the 8-wave tiles (8, 9,
-  // whose fold accumulators spill): 0 is the fastest grouped tile from 3000 to 12032 rows (12032: 154 us against
-  // 206-224 us for 8 and 9).
-  // The int8 256x256 tile runs 16 waves (15) in place of 8 (6), four per SIMD hiding more latency: SILU_Q8's
-  // VALU-heavy epilogue 31.7 -> 30.3 us at config 1; with the grid split into one part per XCD, the bias epilogue too
-  // (config 1 up 22.8 -> 21.9 us, config 0 dense 24.5 -> 24.1 us)
-  // The stage-tiled 2:4 weights (contiguous kilobyte loads) move the balance: there the 8-wave 256x256 tile (10)
-  // beats the 16-wave one (config 1 up 23.9 -> 22.0 us, SILU_Q8 31.4 -> 30.7) and the 16x16 128x128 tile (0) its
-  // 32x32 twin (config 1 down 22.8 -> 22.4 us), alternating runs.
-  static const int order[] = {6, 9, 1, 8, 2, 12, 0, 4, 3, 5, 7};
-  const int64_t want = (int64_t)num_cus() * 64 / 100;
+  // the tile whose model time is least: rounds of workgroups over the CUs, each (c per 128-byte K stage + f)
+  const double stages = p.K / 128.0;
+  const int64_t cus = num_cus();
   int best = -1;
-  for (int id0 : order) {
-    // grouped scales take the 8-wave 128x128 tile (17: 64 tokens x 32 channels a wave, two waves per SIMD) in place
-    // of the 4-wave one: the per-group fold's VALU work of one wave then overlaps the other's matrix instructions
-    // (config-2 feed-forward W2, 3000 x 1280 x 5120 in groups of 256, 2:4: 33.4 -> 29.3 us)
-    const int id = id0 == 6 && !bf ? (p.tiled ? 10 : 15) : (id0 == 0 && grouped ? 17 : id0);
-    if (!fits(id) || (grouped && (id == 12 || id == 8 || id == 9)) || (p.tiled && id == 12)) continue;
-    if (tiles_of(id) >= want) return id;
-    if (best < 0 || tiles_of(id) > tiles_of(best)) best = id;
+  double least = 0.0;
+  const TileCost* table = grouped ? GROUPED_COST : p.E ? SPARSE_COST : DENSE_COST;
+  const size_t n_costs = grouped  ? sizeof(GROUPED_COST) / sizeof(TileCost)
+                         : p.E    ? sizeof(SPARSE_COST) / sizeof(TileCost)
+                                  : sizeof(DENSE_COST) / sizeof(TileCost);
+  for (size_t k = 0; k < n_costs; ++k) {
+    const TileCost& t = table[k];
+    if (!fits(t.id) || (p.E && !p.tiled && t.id == 10)) continue;
+    const int64_t n = (int64_t)((p.M + TILES[t.id].bm - 1) / TILES[t.id].bm) * (p.N / TILES[t.id].bn);
+    const double rounds = t.per_cu == 1  ? (double)((n + cus - 1) / cus)
+                          : n <= cus     ? 1.0
+                          : n <= 2 * cus ? 1.25
+                                         : (double)((n + 2 * cus - 1) / (2 * cus));
+    const double us = rounds * (t.c * stages + t.f + (p.epi == EPI_SILU_Q8 ? t.q8 : 0.0));
+    if (best < 0 || us < least) best = t.id, least = us;
   }
   return best;
 }
