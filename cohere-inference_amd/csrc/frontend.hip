@@ -15,6 +15,7 @@
 #include "common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -206,8 +207,9 @@ __global__ void __launch_bounds__(FPW * 64) logmel_kernel(const float* __restric
 // (only past NKEEP * 512 frames, 30.7 s, are they read again). 16 bands of 16 frames in flight, read three times over,
 // took 101 us there, this 15 us. The 16 workgroups of a piece run on one XCD (contiguous items of the remapped
 // index), whose L2 then merges their 16-byte parts of each output row.
-// four floats / four bf16 values, read or written whole at their own alignment
+// four floats, two or four bf16 values, read or written whole at their own alignment
 typedef float f4_any __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32_any __attribute__((aligned(2)));
 typedef uint32_t b4_any __attribute__((ext_vector_type(2), aligned(2)));
 constexpr int NB = 8, NQ = NB / 4, NTHR = 1024, NFR = NTHR / NQ, NKEEP = 6;
 __global__ void __launch_bounds__(NTHR) normalize_kernel(const float* __restrict__ logmel,
@@ -365,6 +367,255 @@ __global__ void __launch_bounds__(1024) sub_conv0_dw_kernel(const uint16_t* __re
   for (int i = 0; i < SUB_F2; ++i) o[(int64_t)i * C] = f2bf(acc[i]);
 }
 
+// The pointwise convolution of POS positions x 256 channels held in LDS (bf16, rows of 512 bytes, 16-byte chunk c of
+// position r at c ^ (r & 15)): out = relu(bf16(sum) + bias), as the bf16 GEMM's CONV_RELU computes it -- the same
+// matrix instruction, operand roles and K order, so the same bits. NW waves of 256 / NW output channels; the weights go
+// straight from L2 into registers, two K steps ahead. The results replace the operand in LDS and leave as whole rows.
+constexpr int PW_C = 256;
+DEVI int pw_slot(int r, int c) { return r * (2 * PW_C) + ((c ^ (r & 15)) << 4); }  // byte offset of chunk c
+
+template <int POS, int NW>
+DEVI void pointwise(char* tile, const uint16_t* __restrict__ w, const uint16_t* __restrict__ bias,
+                    uint16_t* __restrict__ out, int64_t n_pos) {
+  constexpr int MI = POS / 16, NI = 16 / NW, KS = PW_C / 32;
+  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id(), c16 = lane & 15, h = lane >> 4;
+  const int n0 = wave * (16 * NI);
+  v8bf wf[3][NI];
+  auto load_w = [&](int b, int ks) {
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+      wf[b][j] = *reinterpret_cast<const v8bf*>(w + (n0 + j * 16 + c16) * PW_C + ks * 32 + 8 * h);
+  };
+  load_w(0, 0);
+  load_w(1, 1);
+  uint2 braw[NI];
+#pragma unroll
+  for (int j = 0; j < NI; ++j) braw[j] = *reinterpret_cast<const uint2*>(bias + n0 + j * 16 + 4 * h);
+  v4f acc[NI][MI];
+#pragma unroll
+  for (int j = 0; j < NI; ++j)
+#pragma unroll
+    for (int i = 0; i < MI; ++i) acc[j][i] = v4f{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();  // the tile
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    if (ks + 2 < KS) load_w((ks + 2) % 3, ks + 2);
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const v8bf x = *reinterpret_cast<const v8bf*>(tile + pw_slot(i * 16 + c16, ks * 4 + h));
+#pragma unroll
+      for (int j = 0; j < NI; ++j) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks % 3][j], x, acc[j][i], 0, 0, 0);
+    }
+  }
+  __syncthreads();  // every wave has read the operand
+#pragma unroll
+  for (int j = 0; j < NI; ++j) {
+    const float b4[4] = {__uint_as_float(braw[j].x << 16), __uint_as_float(braw[j].x & 0xffff0000u),
+                         __uint_as_float(braw[j].y << 16), __uint_as_float(braw[j].y & 0xffff0000u)};
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      float v[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = fmaxf(round_bf(acc[j][i][k]) + b4[k], 0.f);
+      const int col = n0 + j * 16 + 4 * h;  // four channels: half of a 16-byte chunk
+      *reinterpret_cast<uint2*>(tile + pw_slot(i * 16 + c16, col >> 3) + (col & 4) * 2) =
+          make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < POS * 32; i += NW * 64) {
+    const int r = i >> 5, c = i & 31;
+    if (r < n_pos)
+      *reinterpret_cast<uint4*>(out + (int64_t)r * PW_C + c * 8) = *reinterpret_cast<const uint4*>(tile + pw_slot(r, c));
+  }
+}
+
+// The same two convolutions and the pointwise one that follows, for C = 256, SUB_T output rows (sequence, t2) per
+// workgroup. On the vector units a conv0 value takes 9 multiply-adds and 7 more instructions, and that issue is all of
+// the kernel above (129 us for 8 pieces of 30 s; with conv0 rows shared between output rows and the pointwise
+// convolution behind it 153). So conv0 runs on the matrix cores: a bf16 mel value and a third of a weight's bits are
+// exact factors, and a weight is the exact sum of three bf16 values (its leading, middle and last 8 bits), so one
+// K = 32 instruction holds the 27 products of a 3 x 3 patch and adds them in fp32 (stem of 8 pieces of 30 s against 64
+// bits: 4.8e-3 either way). Everything after the sum is as above, in the same order. 8 pieces of 30 s: 113 us for what
+// the two launches took 180; what is left is the vector work after the sums (about 60 us) and the phases' latencies.
+//  * A operand: the patches of one conv0 row, 64 positions x 32 K values, gathered in LDS one row ahead of their use
+//    (K index 9 q + tap: tap value for weight part q). Row m of block pb is position 16 (m / 4) + 4 pb + m % 4, so a
+//    lane holds 16 consecutive positions of a channel and the depthwise taps need one value from another lane.
+//  * Where the next row of the list is t2 + 1 of the same sequence (the stem's lists), conv0 row 2 t2 + 1 is computed
+//    once and added to both rows' sums.
+//  * The rows stay in LDS as the pointwise convolution's operand; only its output is written.
+constexpr int SUB_T = 4, SUB_W = 8, SUB_J = 16 / SUB_W;  // output rows, waves, 16-channel blocks of a wave
+constexpr int MEL_LD = MELS + 8, PATCH = 64 * 64;         // patch bytes of a conv0 row
+__global__ void __launch_bounds__(SUB_W * 64) __attribute__((amdgpu_waves_per_eu(4))) sub_conv0_dw_pw_kernel(
+    const uint16_t* __restrict__ feats, int64_t ld_seq, const int* __restrict__ mel_len, const int* __restrict__ rows,
+    int n_rows, const float* __restrict__ w0, const float* __restrict__ b0, const float* __restrict__ w2,
+    const float* __restrict__ b2, const uint16_t* __restrict__ wp, const uint16_t* __restrict__ bp,
+    uint16_t* __restrict__ out) {
+  __shared__ __attribute__((aligned(16))) char tile[SUB_T * SUB_F2 * 2 * PW_C];
+  __shared__ __attribute__((aligned(16))) char patch[2][PATCH];
+  __shared__ uint16_t mel[SUB_T][7][MEL_LD];  // mel rows 4 t2 - 3 .. 4 t2 + 3, column c at c + 1, zeros outside
+  const int tid = threadIdx.x, lane = lane_id(), wave = wave_id(), c16 = lane & 15, h = lane >> 4;
+  const int i0 = blockIdx.x * SUB_T, nt = min(SUB_T, n_rows - i0);
+  // one thread per pair of columns of the seven rows, every load unguarded (a row outside the sequence loads row 0)
+  static_assert(7 * (MELS / 2) <= SUB_W * 64 && SUB_T * 7 * (MEL_LD - MELS) <= SUB_W * 64, "one pass");
+  const int mr = min(tid / (MELS / 2), 6), mc = tid % (MELS / 2) * 2;
+  uint32_t mv[SUB_T];
+#pragma unroll
+  for (int k = 0; k < SUB_T; ++k) {
+    const int i = min(i0 + k, n_rows - 1), seq = rows[2 * i], r = 4 * rows[2 * i + 1] - 3 + mr;
+    const bool in = r >= 0 && r < mel_len[seq];
+    const u32_any v = *reinterpret_cast<const u32_any*>(feats + (int64_t)seq * ld_seq + (in ? (int64_t)r * MELS : 0) + mc);
+    mv[k] = in ? (uint32_t)v : 0u;
+  }
+  // this lane's channels (wave * SUB_J + j) * 16 + c16: conv0 weights as the B operand (K 8 h .. 8 h + 7), depthwise taps
+  v8bf wf[SUB_J];
+  float kd[SUB_J][9], bias0[SUB_J], bias2[SUB_J];
+#pragma unroll
+  for (int j = 0; j < SUB_J; ++j) {
+    const int c = (wave * SUB_J + j) * 16 + c16;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int kk = 8 * h + e, q = kk / 9;
+      float w = w0[c * 9 + kk % 9];
+      const bool finite = __builtin_isfinite(w);
+      // part q of the weight: the 8 leading bits of what the parts before it leave (by truncation: each part exact); an
+      // infinity or NaN is its first part
+      float part = 0.f;
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        part = i <= q ? __uint_as_float(__float_as_uint(w) & 0xffff0000u) : part;
+        w = i < q ? w - part : w;
+      }
+      wf[j][e] = __builtin_bit_cast(__bf16, (uint16_t)(__float_as_uint(kk < 27 && (finite || q == 0) ? part : 0.f) >> 16));
+    }
+#pragma unroll
+    for (int i = 0; i < 9; ++i) kd[j][i] = w2[c * 9 + i];
+    bias0[j] = b0[c];
+    bias2[j] = b2[c];
+  }
+  // the patch values this thread gathers: position f1 of A row tid / 8, K values 4 (tid % 8) .. + 3
+  static_assert(SUB_W == 8, "one thread per 4 K values of a position");
+  const int pm = tid >> 3, pq = tid & 7, f1 = 16 * ((pm & 15) >> 2) + 4 * (pm >> 4) + (pm & 3);
+  // from the patch's first mel value; the 5 spare K values are zero, and so is an infinity or NaN beside the second and
+  // third weight parts (which may be zero)
+  int off[4];
+  uint32_t drop[4];  // exponent bits whose presence in full makes the value zero
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int kk = 4 * pq + e, tap = kk % 9;
+    off[e] = kk < 27 ? tap / 3 * MEL_LD + tap % 3 : 0;
+    drop[e] = kk < 9 ? 0x10000u : kk < 27 ? 0x7f80u : 0u;
+  }
+  auto gather = [&](int b, int k, int r) {  // conv0 row of tap row r of output row k
+    const uint16_t* src = &mel[k][2 * r][2 * f1];
+    uint32_t v[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      uint32_t lo = src[off[2 * e]], hi = src[off[2 * e + 1]];
+      lo = (lo & drop[2 * e]) == drop[2 * e] ? 0u : lo;
+      hi = (hi & drop[2 * e + 1]) == drop[2 * e + 1] ? 0u : hi;
+      v[e] = lo | hi << 16;
+    }
+    *reinterpret_cast<uint2*>(patch[b] + pm * 64 + (((pq >> 1) ^ ((pm >> 2) & 3)) << 4) + (pq & 1) * 8) =
+        make_uint2(v[0], v[1]);
+  };
+  float acc[SUB_J][8], acc2[SUB_J][8];  // depthwise sums of this lane's channels at f2 = 8 h + o, this output row's and the next's
+  // one conv0 row added as tap row r (and, both, to the next output row as tap row 0)
+  auto conv_row = [&](int b, int r, bool both) {
+    v8bf a[4];
+#pragma unroll
+    for (int pb = 0; pb < 4; ++pb)
+      a[pb] = *reinterpret_cast<const v8bf*>(patch[b] + (pb * 16 + c16) * 64 + ((h ^ (c16 >> 2)) << 4));
+#pragma unroll
+    for (int j = 0; j < SUB_J; ++j) {
+      float v[16];
+#pragma unroll
+      for (int pb = 0; pb < 4; ++pb) {
+        const v4f d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pb], wf[j], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+          const uint32_t u = pack_bf2(d[2 * q], d[2 * q + 1]);  // rounded, then the bias, ReLU and the second rounding
+          v[4 * pb + 2 * q] = round_bf_valu(fmaxf(__uint_as_float(u << 16) + bias0[j], 0.f));
+          v[4 * pb + 2 * q + 1] = round_bf_valu(fmaxf(__uint_as_float(u & 0xffff0000u) + bias0[j], 0.f));
+        }
+      }
+      // position 16 h - 1: the last one of the lane 16 below (none for h = 0)
+      const float left = __shfl(v[15], (lane - 16) & 63, 64);
+      const float t0 = r == 0 ? kd[j][0] : r == 1 ? kd[j][3] : kd[j][6], t1 = r == 0 ? kd[j][1] : r == 1 ? kd[j][4] : kd[j][7],
+                  t2 = r == 0 ? kd[j][2] : r == 1 ? kd[j][5] : kd[j][8];
+      auto add = [&](float (&s)[8], float k0, float k1, float k2) {
+#pragma unroll
+        for (int o = 0; o < 8; ++o) {
+          if (o == 0) {
+            const float x = __builtin_fmaf(k0, left, s[0]);
+            s[0] = h > 0 ? x : s[0];
+          } else {
+            s[o] = __builtin_fmaf(k0, v[2 * o - 1], s[o]);
+          }
+          s[o] = __builtin_fmaf(k1, v[2 * o], s[o]);
+          s[o] = __builtin_fmaf(k2, v[2 * o + 1], s[o]);
+        }
+      };
+      add(acc[j], t0, t1, t2);
+      if (both) add(acc2[j], kd[j][0], kd[j][1], kd[j][2]);
+    }
+  };
+  auto clear = [&](float (&s)[SUB_J][8]) {
+#pragma unroll
+    for (int j = 0; j < SUB_J; ++j)
+#pragma unroll
+      for (int o = 0; o < 8; ++o) s[j][o] = bias2[j];
+  };
+  auto follows = [&](int k) {  // output row k + 1 is the next one of the same sequence
+    return k + 1 < nt && rows[2 * (i0 + k) + 2] == rows[2 * (i0 + k)] &&
+           rows[2 * (i0 + k) + 3] == rows[2 * (i0 + k) + 1] + 1;
+  };
+  if (tid < 7 * (MELS / 2)) {
+#pragma unroll
+    for (int k = 0; k < SUB_T; ++k) {
+      mel[k][mr][mc + 1] = (uint16_t)mv[k];
+      mel[k][mr][mc + 2] = (uint16_t)(mv[k] >> 16);
+    }
+  }
+  if (tid < SUB_T * 7 * (MEL_LD - MELS)) {  // the zero columns
+    const int row = tid / (MEL_LD - MELS), e = tid % (MEL_LD - MELS);
+    mel[row / 7][row % 7][e == 0 ? 0 : MELS + e] = 0;
+  }
+  __syncthreads();  // mel rows
+  gather(0, 0, 0);
+  __syncthreads();
+  bool carried = false;  // acc holds this row's tap row 0
+  int b = 0;
+  clear(acc);
+  for (int k = 0; k < nt; ++k) {
+    const int seq = rows[2 * (i0 + k)], t2 = rows[2 * (i0 + k) + 1], T1 = (mel_len[seq] - 1) / 2 + 1;
+    const bool next = follows(k);
+    for (int r = carried ? 1 : 0; r < 3; ++r) {
+      // gather the row that comes after this one: the next tap row, or the next output row's first
+      if (r < 2) gather(b ^ 1, k, r + 1);
+      else if (k + 1 < nt) gather(b ^ 1, k + 1, next ? 1 : 0);
+      const int t1 = 2 * t2 - 1 + r;
+      if (r == 2 && next) clear(acc2);
+      if (t1 >= 0 && t1 < T1) conv_row(b, r, r == 2 && next);
+      __syncthreads();  // the next patches are written, these are read
+      b ^= 1;
+    }
+#pragma unroll
+    for (int j = 0; j < SUB_J; ++j)
+#pragma unroll
+      for (int o = 0; o < 8; ++o) {
+        const int c = (wave * SUB_J + j) * 16 + c16;
+        *reinterpret_cast<uint16_t*>(tile + pw_slot(k * SUB_F2 + 8 * h + o, c >> 3) + (c & 7) * 2) = f2bf(acc[j][o]);
+      }
+    carried = next;
+#pragma unroll
+    for (int j = 0; j < SUB_J; ++j)
+#pragma unroll
+      for (int o = 0; o < 8; ++o) acc[j][o] = next ? acc2[j][o] : bias2[j];
+  }
+  pointwise<SUB_T * SUB_F2, SUB_W>(tile, wp, bp, out + (int64_t)i0 * SUB_F2 * PW_C, (int64_t)nt * SUB_F2);
+}
+
 // depthwise 3x3 stride-2 convolution + bias on channels-last sequences x [sum T_in, F_in, C]: output row
 // (sequence, t) = rows[i] into out [n, F_in / 2, C]; a thread per (row, frequency, 8 channels)
 __global__ void __launch_bounds__(256) sub_dw_kernel(const uint16_t* __restrict__ x, const int* __restrict__ in_start,
@@ -424,6 +675,71 @@ __global__ void __launch_bounds__(256) sub_dw_kernel(const uint16_t* __restrict_
   *reinterpret_cast<uint4*>(out + ((int64_t)i * F_out + fo) * C + c) = o;
 }
 
+// The same depthwise convolution and the pointwise one that follows, for F_in = 32 and C = 256: a workgroup takes DWP_T
+// output rows x 16 frequencies. A thread keeps its 8 channels' 72 taps for 8 outputs (sub_dw_kernel reads them, 320
+// bytes, for each output of 144 input bytes) and two neighbouring frequencies share a column of inputs. 8 pieces of
+// 30 s: 33 us for what the two launches took 58.
+constexpr int DWP_T = 4, DWP_F = 16;
+__global__ void __launch_bounds__(256) sub_dw_pw_kernel(const uint16_t* __restrict__ x, const int* __restrict__ in_start,
+                                                        const int* __restrict__ in_len, const int* __restrict__ rows,
+                                                        const float* __restrict__ w, const float* __restrict__ b,
+                                                        const uint16_t* __restrict__ wp, const uint16_t* __restrict__ bp,
+                                                        uint16_t* __restrict__ out, int n_rows) {
+  __shared__ __attribute__((aligned(16))) char tile[DWP_T * DWP_F * 2 * PW_C];
+  constexpr int F_in = 2 * DWP_F;
+  const int i0 = blockIdx.x * DWP_T, nt = min(DWP_T, n_rows - i0), chunk = threadIdx.x & 31, pl = threadIdx.x >> 5;
+  const int c = chunk * 8, f0 = 4 * pl - 1;  // outputs 2 pl, 2 pl + 1 read input frequencies f0 .. f0 + 4
+  float wk[8 * 9], bias[8];
+#pragma unroll
+  for (int v = 0; v < 18; ++v)
+    *reinterpret_cast<float4*>(wk + 4 * v) = *reinterpret_cast<const float4*>(w + c * 9 + 4 * v);
+  *reinterpret_cast<float4*>(bias) = *reinterpret_cast<const float4*>(b + c);
+  *reinterpret_cast<float4*>(bias + 4) = *reinterpret_cast<const float4*>(b + c + 4);
+  for (int k = 0; k < nt; ++k) {
+    const int seq = rows[2 * (i0 + k)], t = rows[2 * (i0 + k) + 1], start = in_start[seq], len = in_len[seq];
+    float acc[2][8];
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[o][e] = bias[e];
+    uint4 u[3][5];
+#pragma unroll
+    for (int di = 0; di < 3; ++di) {
+      const int ti = 2 * t - 1 + di;  // for a row outside the sequence row 0 is loaded and not used
+      const int64_t row = ti >= 0 && ti < len ? (int64_t)start + ti : 0;
+#pragma unroll
+      for (int dj = 0; dj < 5; ++dj)
+        u[di][dj] = *reinterpret_cast<const uint4*>(x + (row * F_in + max(f0 + dj, 0)) * PW_C + c);
+    }
+    // the taps in order, missing ones skipped (not added as zeros)
+#pragma unroll
+    for (int di = 0; di < 3; ++di) {
+      const int ti = 2 * t - 1 + di;
+      if (ti < 0 || ti >= len) continue;
+#pragma unroll
+      for (int o = 0; o < 2; ++o)
+#pragma unroll
+        for (int dj = 0; dj < 3; ++dj) {
+          const uint4 v = u[di][2 * o + dj];
+          const uint32_t q[4] = {v.x, v.y, v.z, v.w};
+          const bool in = o > 0 || dj > 0 || f0 >= 0;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float xv = __uint_as_float(e & 1 ? q[e / 2] & 0xffff0000u : q[e / 2] << 16);
+            const float s = __builtin_fmaf(wk[e * 9 + di * 3 + dj], xv, acc[o][e]);
+            acc[o][e] = in ? s : acc[o][e];
+          }
+        }
+    }
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+      *reinterpret_cast<uint4*>(tile + pw_slot(k * DWP_F + 2 * pl + o, chunk)) =
+          make_uint4(pack_bf2(acc[o][0], acc[o][1]), pack_bf2(acc[o][2], acc[o][3]), pack_bf2(acc[o][4], acc[o][5]),
+                     pack_bf2(acc[o][6], acc[o][7]));
+  }
+  pointwise<DWP_T * DWP_F, 4>(tile, wp, bp, out + (int64_t)i0 * DWP_F * PW_C, (int64_t)nt * DWP_F);
+}
+
 bool aligned(const void* q, int a) { return (reinterpret_cast<uintptr_t>(q) % a) == 0; }
 
 }  // namespace
@@ -479,4 +795,34 @@ extern "C" int cohere_sub_dw(const uint16_t* x, const int32_t* in_start, const i
   sub_dw_kernel<<<(unsigned)((total + 255) / 256), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
       x, in_start, in_len, rows, w, b, out, n_rows, (int)F_in, (int)C);
   return cohere::check_launch("sub_dw");
+}
+
+extern "C" int cohere_sub_conv0_dw_pw(const uint16_t* feats, int64_t ld_seq, const int32_t* mel_len,
+                                      const int32_t* rows, int64_t n_rows, const float* w0, const float* b0,
+                                      const float* w2, const float* b2, const uint16_t* wp, const uint16_t* bp,
+                                      uint16_t* out, void* stream) {
+  cohere::clear_error();
+  COHERE_REQUIRE(n_rows >= 0 && n_rows < (1LL << 30), "sub_conv0_dw_pw: bad row count");
+  if (n_rows == 0) return 0;
+  COHERE_REQUIRE(feats && mel_len && rows && w0 && b0 && w2 && b2 && wp && bp && out, "sub_conv0_dw_pw: null pointer");
+  COHERE_REQUIRE(aligned(wp, 16) && aligned(bp, 8) && aligned(out, 16),
+                 "sub_conv0_dw_pw: the pointwise weights and out must be 16-byte aligned, its bias 8-byte aligned");
+  sub_conv0_dw_pw_kernel<<<(unsigned)((n_rows + SUB_T - 1) / SUB_T), SUB_W * 64, 0, reinterpret_cast<hipStream_t>(stream)>>>(
+      feats, ld_seq, mel_len, rows, (int)n_rows, w0, b0, w2, b2, wp, bp, out);
+  return cohere::check_launch("sub_conv0_dw_pw");
+}
+
+extern "C" int cohere_sub_dw_pw(const uint16_t* x, const int32_t* in_start, const int32_t* in_len, const int32_t* rows,
+                                int64_t n_rows, const float* w, const float* b, const uint16_t* wp, const uint16_t* bp,
+                                uint16_t* out, void* stream) {
+  cohere::clear_error();
+  COHERE_REQUIRE(n_rows >= 0 && n_rows < (1LL << 30), "sub_dw_pw: bad row count");
+  if (n_rows == 0) return 0;
+  COHERE_REQUIRE(x && in_start && in_len && rows && w && b && wp && bp && out, "sub_dw_pw: null pointer");
+  COHERE_REQUIRE(aligned(x, 16) && aligned(out, 16) && aligned(w, 16) && aligned(b, 16) && aligned(wp, 16) &&
+                     aligned(bp, 8),
+                 "sub_dw_pw: x, out, the taps, the biases and the weights must be 16-byte aligned");
+  sub_dw_pw_kernel<<<(unsigned)((n_rows + DWP_T - 1) / DWP_T), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
+      x, in_start, in_len, rows, w, b, wp, bp, out, (int)n_rows);
+  return cohere::check_launch("sub_dw_pw");
 }

@@ -38,7 +38,8 @@ EXPORTS = ("cohere_gemm_i8", "cohere_gemm_sp", "cohere_quantize_rows", "cohere_l
            "cohere_dec_scatter_kv", "cohere_dec_scatter_kv_q8", "cohere_gemm_bf16", "cohere_logmel_workspace_bytes",
            "cohere_logmel_features", "cohere_sub_conv0_dw", "cohere_sub_dw", "cohere_encoder_branch_workspace_bytes",
            "cohere_encoder_layers_noalloc", "cohere_dec_linear_fused", "cohere_dec_pick_embed",
-           "cohere_gemm_sp_tiled", "cohere_pack_24_tiled_bytes", "cohere_pack_24_tiled")
+           "cohere_gemm_sp_tiled", "cohere_pack_24_tiled_bytes", "cohere_pack_24_tiled", "cohere_sub_conv0_dw_pw",
+           "cohere_sub_dw_pw")
 
 
 def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
@@ -77,6 +78,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
         "cohere_logmel_features": [P, P, I64, I64, P, P, P, F, P, I64, P, P],
         "cohere_sub_conv0_dw": [P, I64, P, P, I64, P, P, P, P, P, I64, P],
         "cohere_sub_dw": [P, P, P, P, I64, P, P, P, I64, I64, P],
+        "cohere_sub_conv0_dw_pw": [P, I64, P, P, I64, P, P, P, P, P, P, P, P],
+        "cohere_sub_dw_pw": [P, P, P, P, I64, P, P, P, P, P, P],
         "cohere_encoder_layers": [P, I64, P, I64, P, P, I64, P, P, I64, I64, I64, ctypes.c_double, I32, I32, I32, P,
                                   I64, P, I64, P],
         "cohere_encoder_layers_noalloc": [P, I64, P, I64, P, P, I64, P, P, I64, I64, I64, ctypes.c_double, I32, I32,
@@ -203,6 +206,42 @@ class _Ext:
             return
         self._call("cohere_sub_dw", _ptr(x), _ptr(in_start), _ptr(in_len), _ptr(rows), n, _ptr(w), _ptr(b),
                    _ptr(out), F_in, C, _stream())
+
+    @staticmethod
+    def _pointwise_checks(w, b, out):
+        _check(w.dtype == b.dtype == out.dtype == torch.bfloat16 and tuple(w.shape) == (256, 256) and
+               w.is_contiguous() and b.numel() == 256 and b.is_contiguous() and out.is_contiguous(),
+               "pointwise convolution: contiguous bf16 (256, 256) weights, (256) bias and output")
+
+    def sub_conv0_dw_pw(self, feats, mel_len, rows, w0, b0, w2, b2, wp, bp, out):
+        """sub_conv0_dw, then the stem's pointwise convolution of its output with wp (256, 256) and bp (256) bf16 and
+        ReLU (gemm with EPI_CONV_RELU), in one launch: out (n, 32, 256); the same bits as the two calls."""
+        _check(feats.is_contiguous() and feats.dim() == 3 and feats.shape[2] == 128 and
+               feats.dtype == torch.bfloat16 and w0.shape[0] == 256 and rows.dtype == torch.int32 and
+               rows.is_contiguous() and mel_len.dtype == torch.int32 and
+               all(t.dtype == torch.float32 and t.is_contiguous() for t in (w0, b0, w2, b2)),
+               "sub_conv0_dw_pw: bad arguments")
+        self._pointwise_checks(wp, bp, out)
+        n = rows.shape[0]
+        _check(tuple(out.shape) == (n, 32, 256), "sub_conv0_dw_pw: out (n, 32, 256)")
+        if n == 0:
+            return
+        self._call("cohere_sub_conv0_dw_pw", _ptr(feats), feats.stride(0), _ptr(mel_len), _ptr(rows), n, _ptr(w0),
+                   _ptr(b0), _ptr(w2), _ptr(b2), _ptr(wp), _ptr(bp), _ptr(out), _stream())
+
+    def sub_dw_pw(self, x, in_start, in_len, rows, w, b, wp, bp, out):
+        """sub_dw on x (sum T_in, 32, 256), then the stem's pointwise convolution as sub_conv0_dw_pw: out (n, 16, 256)."""
+        n = rows.shape[0]
+        _check(x.is_contiguous() and x.dim() == 3 and tuple(x.shape[1:]) == (32, 256) and
+               x.dtype == torch.bfloat16 and rows.dtype == torch.int32 and rows.is_contiguous() and
+               in_start.dtype == torch.int32 and in_len.dtype == torch.int32 and w.dtype == torch.float32 and
+               b.dtype == torch.float32 and w.is_contiguous() and b.is_contiguous(), "sub_dw_pw: bad arguments")
+        self._pointwise_checks(wp, bp, out)
+        _check(tuple(out.shape) == (n, 16, 256), "sub_dw_pw: out (n, 16, 256)")
+        if n == 0:
+            return
+        self._call("cohere_sub_dw_pw", _ptr(x), _ptr(in_start), _ptr(in_len), _ptr(rows), n, _ptr(w), _ptr(b),
+                   _ptr(wp), _ptr(bp), _ptr(out), _stream())
 
     # ---- int8 GEMMs (bindings.cpp:41-43, 59-61) ----------------------------------------------------------------------
 

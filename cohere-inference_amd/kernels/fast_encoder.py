@@ -321,17 +321,24 @@ class SubsamplingStem:
         dev, dt, C = features.device, features.dtype, self.c
         quarter, eighth = self.lengths(frames)
         as_dev = lambda v: torch.tensor(v, dtype=torch.int32).to(dev, non_blocking=True)  # noqa: E731
-        # stage 1: (rows at stride 4, 32 frequencies, C) from the log-mel frames of each piece
-        h = torch.empty(sum(quarter), 32, C, device=dev, dtype=dt)
-        ext.sub_conv0_dw(features.contiguous(), as_dev(frames), self._row_index(quarter, dev), *self.first, h)
-        h = gemm(h.view(-1, C), *self.pointwise[0], EPI_CONV_RELU).view(-1, 32, C)
-        # stage 2: depthwise at stride 2 in time and frequency, within each piece's rows of stage 1
+        # stage 1: (rows at stride 4, 32 frequencies, C) from the log-mel frames of each piece; stage 2: depthwise at
+        # stride 2 in time and frequency, within each piece's rows of stage 1. Each is followed by its pointwise
+        # convolution, in the same launch for 256 channels
+        fused = C == 256 and self.freq == 16
         first_row = [0]
         for t in quarter[:-1]:
             first_row.append(first_row[-1] + t)
+        rows1, rows2 = self._row_index(quarter, dev), self._row_index(eighth, dev)
+        h = torch.empty(sum(quarter), 32, C, device=dev, dtype=dt)
         g = torch.empty(sum(eighth), 16, C, device=dev, dtype=dt)
-        ext.sub_dw(h, as_dev(first_row), as_dev(quarter), self._row_index(eighth, dev), *self.second_dw, g)
-        g = gemm(g.view(-1, C), *self.pointwise[1], EPI_CONV_RELU)
+        if fused:
+            ext.sub_conv0_dw_pw(features.contiguous(), as_dev(frames), rows1, *self.first, *self.pointwise[0], h)
+            ext.sub_dw_pw(h, as_dev(first_row), as_dev(quarter), rows2, *self.second_dw, *self.pointwise[1], g)
+        else:
+            ext.sub_conv0_dw(features.contiguous(), as_dev(frames), rows1, *self.first, h)
+            h = gemm(h.view(-1, C), *self.pointwise[0], EPI_CONV_RELU).view(-1, 32, C)
+            ext.sub_dw(h, as_dev(first_row), as_dev(quarter), rows2, *self.second_dw, g)
+            g = gemm(g.view(-1, C), *self.pointwise[1], EPI_CONV_RELU)
         return gemm(g.view(-1, self.freq * C), *self.linear, EPI_BIAS), eighth
 
 

@@ -324,6 +324,20 @@ int cohere_sub_dw(const uint16_t* x, const int32_t* in_start, const int32_t* in_
                   int64_t n_rows, const float* w, const float* b, uint16_t* out, int64_t F_in, int64_t C,
                   void* stream);
 
+/* sub_conv0_dw with 256 channels, then the pointwise convolution that follows it in the stem (reference
+ * kernels/fast_encoder.py:193-199: gemm with CONV_RELU): wp bf16 [256, 256] (output channel, input channel), bp bf16
+ * [256]; out bf16 [n_rows, 32, 256] = relu(bf16(pointwise sum) + bp). The same bits as the two calls. 16-byte aligned
+ * wp and out, 8-byte aligned bp. */
+int cohere_sub_conv0_dw_pw(const uint16_t* feats, int64_t ld_seq, const int32_t* mel_len, const int32_t* rows,
+                           int64_t n_rows, const float* w0, const float* b0, const float* w2, const float* b2,
+                           const uint16_t* wp, const uint16_t* bp, uint16_t* out, void* stream);
+
+/* sub_dw with F_in = 32 and 256 channels, then the pointwise convolution that follows it, as above: out bf16
+ * [n_rows, 16, 256]. */
+int cohere_sub_dw_pw(const uint16_t* x, const int32_t* in_start, const int32_t* in_len, const int32_t* rows,
+                     int64_t n_rows, const float* w, const float* b, const uint16_t* wp, const uint16_t* bp,
+                     uint16_t* out, void* stream);
+
 /* The last error on this thread ("" when none). */
 const char* cohere_last_error(void);
 
