@@ -44,7 +44,10 @@ namespace cohere_gemm {
 // the reference's epilogue ids (kernels/cuda_ext.py:28); RELU and CONV_RELU are bf16-operand only (SILU too through the
 // C ABI; the few-row layers use it on int8 operands), I32 is ours
 enum { EPI_BIAS = 0, EPI_SILU = 1, EPI_RELU = 2, EPI_RESID = 3, EPI_GLU = 4, EPI_SILU_Q8 = 5, EPI_CONV_RELU = 6,
-       EPI_I32 = 7 };
+       EPI_I32 = 7,
+       // internal, bf16 operands: BIAS whose rows go straight into the decoder's cross-attention caches, as
+       // dec_scatter_kv (_q8: int8 with a scale per 128 columns) stores them
+       EPI_KV = 8, EPI_KV8 = 9 };
 
 struct GemmArgs {
   const int8_t* X;       // tokens [M, K], row stride ldx
@@ -64,6 +67,12 @@ struct GemmArgs {
   float alpha;
   int xcd_rows;          // > 0: the token tiles split into xcd_rows parts and the channel tiles into 8 / xcd_rows,
                          // one part each per XCD (set by launch_tile); 0: contiguous tile ranges per XCD
+  // EPI_KV, EPI_KV8: column block c of 128 is layer c / 2H, key (even) or value (odd) c / H % 2, head c % H; caches
+  // (layers, S, H, T, 128) with scales (layers, S, H, T); output row m goes to slot slot_of[m], position frame_of[m]
+  void *kc, *vc;
+  float *ks, *vs;
+  const int32_t *slot_of, *frame_of;
+  int S, H, T;
   int tiled;             // 2:4 only: W holds the stage-tiled layout of the kept values and selectors (E unused)
 };
 
@@ -171,7 +180,9 @@ DEVI int sw64(int r, int c) { return r * 64 + ((c ^ ((r >> 1) & 3)) << 4); }
 template <int BM, int BN, int WM, int WN, int ST, int MS, int EPI, bool GROUPED, bool SPARSE, int GS = 0,
           bool BF = false>
 __global__ void __launch_bounds__(WM* WN * 64) gemm_q8_kernel(const GemmArgs p) {
+  constexpr bool KV = EPI == EPI_KV || EPI == EPI_KV8;
   static_assert(!BF || (!SPARSE && !GROUPED && EPI != EPI_SILU_Q8 && EPI != EPI_I32), "bf16 operands");
+  static_assert(!KV || (BF && BN % 128 == 0), "cache epilogue");
   static_assert(BF || (EPI != EPI_RELU && EPI != EPI_CONV_RELU), "bf16-only epilogue");
   using T = Tile<BM, BN, WM, WN, ST, MS, GROUPED, SPARSE>;
   constexpr int NW = T::NW, NT = T::NT, TM = T::TM, TN = T::TN, MI = T::MI, NI = T::NI, LPS = T::LPS;
@@ -600,7 +611,7 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_q8_kernel(const GemmArgs p) 
       }
     };
     if constexpr (EPI == EPI_BIAS || EPI == EPI_RESID || EPI == EPI_GLU || EPI == EPI_SILU || EPI == EPI_RELU ||
-                  EPI == EPI_CONV_RELU) {
+                  EPI == EPI_CONV_RELU || KV) {
       // the tile's bf16 results are staged in LDS (over the pipeline buffers, free now) and written out as whole
       // rows: each 16-byte store then covers 8 consecutive channels of one row, where the lanes' own results would
       // give 16 rows x 8 bytes per instruction. A row's 8-byte units (4 channels) are XOR-swizzled by the row's low
@@ -663,7 +674,29 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_q8_kernel(const GemmArgs p) 
                                              __uint_as_float(rr[k] & 0xffff0000u)));
           o = make_uint4(res[0], res[1], res[2], res[3]);
         }
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.C) + (int64_t)m * p.ldc + oc0 + cc * 8) = o;
+        if constexpr (KV) {
+          // the chunk's 128-vector: 16 consecutive lanes of one row hold it (m is theirs together)
+          const int cb = (oc0 >> 7) + (cc >> 4), d8 = cc & 15, hd = cb % p.H, kvi = cb / p.H % 2, l = cb / p.H / 2;
+          const int64_t vec = (((int64_t)l * p.S + p.slot_of[m]) * p.H + hd) * p.T + p.frame_of[m];
+          if constexpr (EPI == EPI_KV) {
+            *reinterpret_cast<uint4*>(static_cast<uint16_t*>(kvi ? p.vc : p.kc) + vec * 128 + d8 * 8) = o;
+          } else {
+            const uint32_t ov[4] = {o.x, o.y, o.z, o.w};
+            float f[8], mx = 0.f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              f[k] = __uint_as_float(k & 1 ? ov[k >> 1] & 0xffff0000u : ov[k >> 1] << 16);
+              mx = fmaxf(mx, fabsf(f[k]));
+            }
+            mx = row16_max(mx);
+            const float sc = mx > 0.f ? mx / 127.f : 1.f, inv = 1.f / sc;
+            *reinterpret_cast<uint2*>(static_cast<int8_t*>(kvi ? p.vc : p.kc) + vec * 128 + d8 * 8) =
+                make_uint2(q8x4(f[0], f[1], f[2], f[3], inv), q8x4(f[4], f[5], f[6], f[7], inv));
+            if (d8 == 0) (kvi ? p.vs : p.ks)[vec] = sc;
+          }
+        } else {
+          *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.C) + (int64_t)m * p.ldc + oc0 + cc * 8) = o;
+        }
       }
     } else if constexpr (EPI == EPI_SILU_Q8) {
       // u = bf16(silu(bf16(v))), kept (as float bits) in the accumulator registers; the max |u| of each (row,

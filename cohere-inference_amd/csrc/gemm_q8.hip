@@ -51,6 +51,7 @@ int choose_tile(const GemmArgs& p, bool grouped, bool bf = false) {
   auto fits = [&](int id) {
     const TileInfo& t = TILES[id];
     if (bf && !bf16_tile(id)) return false;
+    if ((p.epi == EPI_KV || p.epi == EPI_KV8) && (t.bn % 128 || id == 8)) return false;
     if (p.N % t.bn) return false;
     if (grouped && !t.grouped_ok) return false;
     if (p.epi == EPI_SILU_Q8 && t.bn % p.qgroup) return false;
@@ -257,4 +258,49 @@ extern "C" int cohere_gemm_bf16(const uint16_t* a, int64_t lda, const uint16_t* 
     return 1;
   }
   return cohere::check_launch("gemm");
+}
+
+namespace {
+int gemm_kv_entry(bool q8, const uint16_t* a, int64_t lda, const uint16_t* w, const uint16_t* bias, int64_t M, int64_t K,
+                  const int32_t* slot_of, const int32_t* frame_of, void* ck, void* cv, float* cks, float* cvs, int64_t L,
+                  int64_t S, int64_t H, int64_t T, void* stream, const char* name) {
+  const std::string nm(name);
+  COHERE_REQUIRE(M >= 0 && K > 0 && M < (1LL << 31) && K < (1LL << 30) && L > 0 && S > 0 && H > 0 && T > 0 &&
+                     L * H < (1LL << 22) && S < (1LL << 31) && T < (1LL << 31),
+                 nm + ": bad sizes");
+  COHERE_REQUIRE(K % 32 == 0, nm + ": K must be a multiple of 32");
+  COHERE_REQUIRE(a && w && slot_of && frame_of && ck && cv && (!q8 || (cks && cvs)), nm + ": null pointer");
+  COHERE_REQUIRE(lda % 8 == 0 && aligned16(a) && aligned16(w), nm + ": operand rows must be 16-byte aligned");
+  COHERE_REQUIRE(!bias || (reinterpret_cast<uintptr_t>(bias) & 7) == 0, nm + ": bias must be 8-byte aligned");
+  COHERE_REQUIRE(aligned16(ck) && aligned16(cv), nm + ": caches must be 16-byte aligned");
+  if (M == 0) return 0;
+  GemmArgs p{};
+  p.X = reinterpret_cast<const int8_t*>(a); p.W = reinterpret_cast<const int8_t*>(w); p.bias = bias;
+  p.ldx = 2 * lda; p.M = (int)M; p.N = (int)(L * 2 * H * 128); p.K = (int)(2 * K); p.group = p.K; p.qgroup = 256;
+  p.alpha = 1.f; p.epi = q8 ? EPI_KV8 : EPI_KV; p.kc = ck; p.vc = cv; p.ks = cks; p.vs = cvs; p.slot_of = slot_of;
+  p.frame_of = frame_of; p.S = (int)S; p.H = (int)H; p.T = (int)T;
+  const int tile = choose_tile(p, false, true);
+  COHERE_REQUIRE(tile >= 0, nm + ": no gfx950 tile fits");
+  if (!launch_gemm_bf16(tile, p.epi, p, reinterpret_cast<hipStream_t>(stream))) {
+    cohere::set_error(nm + ": tile " + std::to_string(tile) + " has no cache epilogue");
+    return 1;
+  }
+  return cohere::check_launch(name);
+}
+}  // namespace
+
+extern "C" int cohere_gemm_kv(const uint16_t* a, int64_t lda, const uint16_t* w, const uint16_t* bias, int64_t M,
+                              int64_t K, const int32_t* slot_of, const int32_t* frame_of, uint16_t* ck, uint16_t* cv,
+                              int64_t L, int64_t S, int64_t H, int64_t T, void* stream) {
+  cohere::clear_error();
+  return gemm_kv_entry(false, a, lda, w, bias, M, K, slot_of, frame_of, ck, cv, nullptr, nullptr, L, S, H, T, stream,
+                       "gemm_kv");
+}
+
+extern "C" int cohere_gemm_kv_q8(const uint16_t* a, int64_t lda, const uint16_t* w, const uint16_t* bias, int64_t M,
+                                 int64_t K, const int32_t* slot_of, const int32_t* frame_of, int8_t* ck, int8_t* cv,
+                                 float* cks, float* cvs, int64_t L, int64_t S, int64_t H, int64_t T, void* stream) {
+  cohere::clear_error();
+  return gemm_kv_entry(true, a, lda, w, bias, M, K, slot_of, frame_of, ck, cv, cks, cvs, L, S, H, T, stream,
+                       "gemm_kv_q8");
 }

@@ -39,7 +39,7 @@ EXPORTS = ("cohere_gemm_i8", "cohere_gemm_sp", "cohere_quantize_rows", "cohere_l
            "cohere_logmel_features", "cohere_sub_conv0_dw", "cohere_sub_dw", "cohere_encoder_branch_workspace_bytes",
            "cohere_encoder_layers_noalloc", "cohere_dec_linear_fused", "cohere_dec_pick_embed",
            "cohere_gemm_sp_tiled", "cohere_pack_24_tiled_bytes", "cohere_pack_24_tiled", "cohere_sub_conv0_dw_pw",
-           "cohere_sub_dw_pw")
+           "cohere_sub_dw_pw", "cohere_gemm_kv", "cohere_gemm_kv_q8")
 
 
 def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
@@ -80,6 +80,8 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
         "cohere_sub_dw": [P, P, P, P, I64, P, P, P, I64, I64, P],
         "cohere_sub_conv0_dw_pw": [P, I64, P, P, I64, P, P, P, P, P, P, P, P],
         "cohere_sub_dw_pw": [P, P, P, P, I64, P, P, P, P, P, P],
+        "cohere_gemm_kv": [P, I64, P, P, I64, I64, P, P, P, P, I64, I64, I64, I64, P],
+        "cohere_gemm_kv_q8": [P, I64, P, P, I64, I64, P, P, P, P, P, P, I64, I64, I64, I64, P],
         "cohere_encoder_layers": [P, I64, P, I64, P, P, I64, P, P, I64, I64, I64, ctypes.c_double, I32, I32, I32, P,
                                   I64, P, I64, P],
         "cohere_encoder_layers_noalloc": [P, I64, P, I64, P, P, I64, P, P, I64, I64, I64, ctypes.c_double, I32, I32,
@@ -570,6 +572,32 @@ class _Ext:
                "dec_scatter_kv_q8: shapes")
         self._call("cohere_dec_scatter_kv_q8", _ptr(kv), kv.shape[0], _ptr(slot_of), _ptr(frame_of), _ptr(ck),
                    _ptr(cv), _ptr(cks), _ptr(cvs), L, S, H, T, _stream())
+
+
+    def gemm_kv(self, a, w, bias, slot_of, frame_of, ck, cv, cks=None, cvs=None):
+        """The cross-attention key and value projections of packed frames a (rows, K) with every layer's weights w
+        (L 2 H 128, K), straight into the slots' caches: gemm with EPI_BIAS, then dec_scatter_kv (dec_scatter_kv_q8 with
+        the scales cks, cvs), in one launch; the same bytes."""
+        L, S, H, T = ck.shape[:4]
+        kind = torch.bfloat16 if cks is None else torch.int8
+        _check(a.dtype == w.dtype == torch.bfloat16 and (bias is None or bias.dtype == torch.bfloat16), "gemm_kv: bf16 only")
+        _check(a.dim() == 2 and w.dim() == 2 and a.stride(1) == 1 and w.is_contiguous() and a.shape[1] == w.shape[1] and
+               a.shape[1] % 32 == 0 and w.shape[0] == L * 2 * H * 128, "gemm_kv: operand shapes")
+        _check(ck.dtype == cv.dtype == kind and ck.is_contiguous() and cv.is_contiguous() and ck.shape == cv.shape and
+               ck.shape[4] == 128, "gemm_kv: caches (L, S, H, T, 128) contiguous")
+        _check(slot_of.dtype == frame_of.dtype == torch.int32 and slot_of.numel() >= a.shape[0] and
+               frame_of.numel() >= a.shape[0] and slot_of.is_contiguous() and frame_of.is_contiguous(),
+               "gemm_kv: int32 slot and frame per row")
+        if a.shape[0] == 0:
+            return
+        if cks is None:
+            self._call("cohere_gemm_kv", _ptr(a), a.stride(0), _ptr(w), _ptr(bias), a.shape[0], a.shape[1],
+                       _ptr(slot_of), _ptr(frame_of), _ptr(ck), _ptr(cv), L, S, H, T, _stream())
+        else:
+            _check(cks.dtype == cvs.dtype == torch.float32 and cks.is_contiguous() and cvs.is_contiguous(),
+                   "gemm_kv: fp32 scales")
+            self._call("cohere_gemm_kv_q8", _ptr(a), a.stride(0), _ptr(w), _ptr(bias), a.shape[0], a.shape[1],
+                       _ptr(slot_of), _ptr(frame_of), _ptr(ck), _ptr(cv), _ptr(cks), _ptr(cvs), L, S, H, T, _stream())
 
 
 _lib = load_library()

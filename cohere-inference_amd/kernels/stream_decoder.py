@@ -377,7 +377,7 @@ class StreamDecoder:
     def fill_cross(self, hidden: torch.Tensor, lengths: list[int], slots: list[int], projected: bool = False) -> None:
         """Cross-attention keys and values of packed encoder frames hidden (sum(lengths), width) into the given slots,
         on the current stream: the decoder's input projection (unless projected), every layer's key and value
-        projections in one bf16 GEMM, then the scatter into the slots' caches (quantized per 128-vector with int8)."""
+        projections in one bf16 GEMM whose epilogue writes the slots' caches (quantized per 128-vector with int8)."""
         from kernels.cuda_ext import EPI_BIAS
 
         rows = hidden.shape[0]
@@ -388,16 +388,12 @@ class StreamDecoder:
             out = torch.empty(rows, self.proj[0].shape[0], device=hidden.device, dtype=hidden.dtype)
             ext.gemm(mem, self.proj[0], self.proj[1], out, EPI_BIAS, None, 1.0, 8)
             mem = out
-        kv = torch.empty(rows, self.cross_w.shape[0], device=hidden.device, dtype=hidden.dtype)
-        ext.gemm(mem, self.cross_w, self.cross_b, kv, EPI_BIAS, None, 1.0, 8)
         where = torch.empty(2, rows, dtype=torch.int32)
         where[0] = torch.repeat_interleave(torch.tensor(slots, dtype=torch.int32), torch.tensor(lengths))
         where[1] = torch.cat([torch.arange(n, dtype=torch.int32) for n in lengths])
         where = where.pin_memory().to(hidden.device, non_blocking=True)
-        if self.int8:
-            ext.dec_scatter_kv_q8(kv, where[0], where[1], self.cross_k, self.cross_v, self.cross_ks, self.cross_vs)
-        else:
-            ext.dec_scatter_kv(kv, where[0], where[1], self.cross_k, self.cross_v)
+        ext.gemm_kv(mem, self.cross_w, self.cross_b, where[0], where[1], self.cross_k, self.cross_v, self.cross_ks,
+                    self.cross_vs)
 
     def admit(self, slots: list[int], prompts: list[torch.Tensor], frames: list[int],
               max_new: list[int] | None = None) -> None:

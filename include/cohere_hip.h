@@ -241,6 +241,18 @@ int cohere_dec_scatter_kv_q8(const uint16_t* kv, int64_t rows, const int32_t* sl
                              int8_t* ck, int8_t* cv, float* cks, float* cvs, int64_t L, int64_t S, int64_t H,
                              int64_t T, void* stream);
 
+/* gemm (bf16, BIAS) of the cross-attention key and value projections with dec_scatter_kv / dec_scatter_kv_q8 as its
+ * epilogue (reference kernels/stream_decoder.py:216-238 runs the two in turn): a bf16 [M, K], w bf16 [L 2 H 128, K]
+ * (per layer the key heads, then the value heads), bias bf16 [L 2 H 128] or null; row i goes to position frame_of[i]
+ * of slot slot_of[i] of the caches (L, S, H, T, 128), int8 with scales (L, S, H, T). The same bytes as the two calls.
+ * K % 32 == 0; 16-byte aligned rows, weights and caches. */
+int cohere_gemm_kv(const uint16_t* a, int64_t lda, const uint16_t* w, const uint16_t* bias, int64_t M, int64_t K,
+                   const int32_t* slot_of, const int32_t* frame_of, uint16_t* ck, uint16_t* cv, int64_t L, int64_t S,
+                   int64_t H, int64_t T, void* stream);
+int cohere_gemm_kv_q8(const uint16_t* a, int64_t lda, const uint16_t* w, const uint16_t* bias, int64_t M, int64_t K,
+                      const int32_t* slot_of, const int32_t* frame_of, int8_t* ck, int8_t* cv, float* cks, float* cvs,
+                      int64_t L, int64_t S, int64_t H, int64_t T, void* stream);
+
 /* Number of per-layer tensors of cohere_encoder_layers: the reference's 53 (its enum F,
  * kernels/csrc/encoder_loop.cpp:34-44) followed by 4 of this library's own (the feed-forwards' first linears in 2:4
  * form: ff1 kept bytes, ff1 selectors, ff2 kept bytes, ff2 selectors; NULL keeps the dense first linear, as the

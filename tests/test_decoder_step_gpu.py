@@ -393,3 +393,27 @@ def test_decoder_built_behind_queued_work(gpu):
     torch.cuda.synchronize()
     for name in ("logits", "tok", "pos", "out", "self_k", "self_v"):
         assert torch.equal(getattr(idle, name), getattr(busy, name)), name
+
+
+@pytest.mark.parametrize("q8", [True, False])
+@pytest.mark.parametrize("rows,L,H", [(1, 1, 1), (70, 2, 3), (400, 3, 8), (1500, 8, 8)])
+def test_gemm_kv_equals_gemm_then_scatter(gpu, rows, L, H, q8):
+    """The projections with the caches' layout as their epilogue against the GEMM and the scatter launched in turn, from
+    the smallest tile to the largest: every byte of the caches and scales, rows in any slot order."""
+    g = torch.Generator().manual_seed(rows + L + H)
+    S, T, K, N = 5, 500, 96, L * 2 * H * 128
+    a = torch.randn(rows, K, generator=g).to(torch.bfloat16).to(gpu)
+    a[rows // 2] = 0  # with no bias: vectors of zeros, scale 1
+    w = (0.1 * torch.randn(N, K, generator=g)).to(torch.bfloat16).to(gpu)
+    where = torch.randperm(S * T, generator=g)[:rows]
+    slot_of, frame_of = (where // T).to(torch.int32).to(gpu), (where % T).to(torch.int32).to(gpu)
+    for bias in (None, torch.randn(N, generator=g).to(torch.bfloat16).to(gpu)):
+        got, want = ([torch.zeros(L, S, H, T, 128, device=gpu, dtype=torch.int8 if q8 else torch.bfloat16)
+                      for _ in range(2)] + ([torch.zeros(L, S, H, T, device=gpu) for _ in range(2)] if q8 else [])
+                     for _ in range(2))
+        kv = torch.empty(rows, N, dtype=torch.bfloat16, device=gpu)
+        _ext().gemm(a, w, bias, kv, 0, None, 1.0, 8)
+        (_ext().dec_scatter_kv_q8 if q8 else _ext().dec_scatter_kv)(kv, slot_of, frame_of, *want)
+        _ext().gemm_kv(a, w, bias, slot_of, frame_of, *got)
+        for x, y in zip(got, want):
+            assert torch.equal(x, y)
