@@ -81,15 +81,19 @@ DEVI v8bf as_bf8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
 // for a block's activations never waits for weights (loads complete in order), and each matrix instruction waits for
 // its own block's weights only. (Conditional loads made the compiler wait for all weights at the branches' join and
 // then fetch each block's activations as a round trip of its own.)
-template <int MB, int NS, int NW, bool W8, int EP, bool LN, int RB = 16, int BPW = 0>
+// CB < 16 (with NS == 1): the strip is CB channels only; the instruction's 16 weight rows repeat them (lanes CB apart
+// load the same addresses) and the repeats are not written. A 1024-wide projection then streams its weights over 256
+// CUs instead of 64, each a quarter of the bytes. A channel's sum keeps its order.
+template <int MB, int NS, int NW, bool W8, int EP, bool LN, int RB = 16, int BPW = 0, int CB = 16>
 __global__ void __launch_bounds__(NW * 64) skinny_kernel(const SkinnyArgs p) {
   static_assert(RB == 16 || (MB == 1 && (RB == 8 || RB == 4)), "row block");
+  static_assert(CB == 16 || (NS == 1 && CB == 4), "channel strip");
   constexpr int ROWS = RB == 16 ? MB * 16 : RB;  // rows per workgroup
   constexpr int MAXB = BPW > 0 ? BPW : (W8 ? 16 : 8) / NS;  // K blocks per wave in registers at once (<= 64 VGPRs)
   static_assert(BPW == 0 || BPW * NS * (W8 ? 1 : 2) <= 16, "weight registers");
   constexpr bool XPRE = BPW > 0 && !LN;  // the activations loaded ahead of the weights
   constexpr bool FULLROW = LN && BPW * NW * KB == LN_K;  // K is the LayerNorm's full 1024: unguarded row loads
-  constexpr int COLS = NS * 16, LDR = COLS + 4;
+  constexpr int COLS = NS * CB, LDR = COLS + 4;
   constexpr int RED = NW * MB * 16 * LDR * 4, XS = LN ? ROWS * LN_ROW : 0;
   // the waves' partial tiles (after the K loop) share LDS with the normalised rows (during it)
   __shared__ __attribute__((aligned(16))) char smem[RED > XS ? RED : XS];
@@ -97,6 +101,7 @@ __global__ void __launch_bounds__(NW * 64) skinny_kernel(const SkinnyArgs p) {
   const int n0 = blockIdx.x * COLS, m_base = blockIdx.y * ROWS;  // grid.y > 1: the rows split over workgroups
   const int lane = threadIdx.x & 63, wave = wave_id(), h = lane >> 4, c16 = lane & 15;
   const int xrow = c16 & (RB - 1);  // the activation row of this lane's matrix column
+  const int wrow = c16 & (CB - 1);  // the channel of this lane's matrix row
   const int nkb = p.K / KB;  // wave w takes blocks w, w + NW, ...
 
   v4f acc[NS][MB];
@@ -152,7 +157,7 @@ __global__ void __launch_bounds__(NW * 64) skinny_kernel(const SkinnyArgs p) {
         const int64_t k = (int64_t)kb * KB;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
-          const int64_t n = n0 + s * 16 + c16;
+          const int64_t n = n0 + s * 16 + wrow;
           if constexpr (W8) {
             wreg[b][s][0] = *reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(p.W) + n * p.K + k + 16 * h);
           } else {
@@ -239,7 +244,7 @@ __global__ void __launch_bounds__(NW * 64) skinny_kernel(const SkinnyArgs p) {
   for (int s = 0; s < NS; ++s)
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb)
-      *reinterpret_cast<v4f*>(&red[wave][mb * 16 + c16][s * 16 + h * 4]) = acc[s][mb];
+      if (CB == 16 || h * 4 < CB) *reinterpret_cast<v4f*>(&red[wave][mb * 16 + c16][s * 16 + h * 4]) = acc[s][mb];
   __syncthreads();
   const int rows = min(p.M - m_base, ROWS);
   for (int i = threadIdx.x; i < rows * COLS; i += NW * 64) {
@@ -272,27 +277,45 @@ int device_cus() {
 
 // the kernel with every wave's loads unconditional when K splits into exactly 2 or 8 blocks per wave (the decoder's
 // 1024 and 4096) and the registers fit; otherwise the general loop
-template <int MB, int NS, int NW, bool W8, int EP, bool LN, int RB = 16>
+template <int MB, int NS, int NW, bool W8, int EP, bool LN, int RB = 16, int CB = 16>
 void launch_k(dim3 grid, const SkinnyArgs& p, hipStream_t s) {
   constexpr int WR = NS * (W8 ? 1 : 2);  // weight registers (x4) per block
   const int nkb = p.K / KB;
   if (nkb == 2 * NW && (LN || MB <= 4)) {
-    skinny_kernel<MB, NS, NW, W8, EP, LN, RB, 2><<<grid, NW * 64, 0, s>>>(p);
+    skinny_kernel<MB, NS, NW, W8, EP, LN, RB, 2, CB><<<grid, NW * 64, 0, s>>>(p);
     return;
   }
   if constexpr (8 * WR <= 16 && MB == 1) {
     if (nkb == 8 * NW) {
-      skinny_kernel<MB, NS, NW, W8, EP, LN, RB, 8><<<grid, NW * 64, 0, s>>>(p);
+      skinny_kernel<MB, NS, NW, W8, EP, LN, RB, 8, CB><<<grid, NW * 64, 0, s>>>(p);
       return;
     }
   }
-  skinny_kernel<MB, NS, NW, W8, EP, LN, RB><<<grid, NW * 64, 0, s>>>(p);
+  skinny_kernel<MB, NS, NW, W8, EP, LN, RB, 0, CB><<<grid, NW * 64, 0, s>>>(p);
 }
 
 template <int NS, int NW, bool W8, int EP, bool LN>
 void launch_rows(const SkinnyArgs& p, hipStream_t s) {
   const int grid = p.N / (NS * 16), mblocks = (p.M + 15) / 16, mblocks8 = (p.M + 7) / 8;
-  if (grid * mblocks < grid * mblocks8 && grid * mblocks8 <= device_cus()) {
+  const int cus = device_cus();
+  if constexpr (LN && NW == 8) {
+    // A LayerNorm prologue at up to 8 rows: 8 rows a workgroup, so each wave normalises one row, not two (4096 x 1024
+    // over 8 rows 5.4 -> 4.1 us, 3072 x 1024 5.2 -> 4.2), and strips of 4 channels while those still find idle CUs
+    // (1024 x 1024 4.8 -> 3.4). Without the prologue narrow strips gained nothing (1024 x 1024 4.8 -> 4.1, but the
+    // whole step no faster) or lost (1024 x 4096 over 8 rows 6.9 -> 8.6: the activations, read by every strip, become
+    // the larger part of the traffic).
+    if (p.M <= 8) {
+      if constexpr (NS == 1) {
+        if (grid * 4 <= cus) {
+          launch_k<1, NS, NW, W8, EP, LN, 8, 4>(dim3(grid * 4), p, s);
+          return;
+        }
+      }
+      launch_k<1, NS, NW, W8, EP, LN, 8>(dim3(grid), p, s);
+      return;
+    }
+  }
+  if (grid * mblocks < grid * mblocks8 && grid * mblocks8 <= cus) {
     // fewer (strip, 16 rows) workgroups than CUs: one workgroup per (strip, 8 rows) instead -- twice the CUs stream
     // the weights, and each fetches half the activations (9-32 rows of the 1024 x 1024 and 1024 x 4096 projections)
     launch_k<1, NS, NW, W8, EP, LN, 8>(dim3(grid, mblocks8), p, s);

@@ -158,6 +158,27 @@ def test_dec_linear_fused_ln_prologue(N, K, w8, relu, M, gpu):
     _check_close(bf16_bits(y), want)
 
 
+@pytest.mark.parametrize("N,K", [(16, 512), (1024, 1024), (1040, 640), (3072, 1024), (8192, 576)])
+@pytest.mark.parametrize("w8", [True, False])
+def test_dec_linear_fused_few_rows_same_bits(N, K, w8, gpu):
+    """1-8 rows take 8-row workgroups (and strips of 4 channels where few): each row has the bits that it has among 16
+    rows, where neither is used; K of 512 and 1024 take the unguarded loads, 576 and 640 the general loop."""
+    from kernels.cuda_ext import DEC_EP_RELU, ext
+    from kernels.stream_decoder import prepare_w8
+
+    x, w, b = linear_inputs(16, N, K, seed=N + K)
+    xg, bg = x.cuda(), b.cuda()
+    wq, sw = (t.cuda() for t in prepare_w8(w)) if w8 else (w.cuda(), None)
+    ln = (torch.rand(K).to(torch.bfloat16).cuda(), torch.rand(K).to(torch.bfloat16).cuda(), 1e-5)
+    full = torch.empty(16, N, dtype=torch.bfloat16, device="cuda")
+    ext.dec_linear_fused(xg, wq, sw, bg, full, DEC_EP_RELU, ln=ln)
+    for M in (1, 3, 7, 8):
+        y = torch.full((M + 1, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        ext.dec_linear_fused(xg[:M], wq, sw, bg, y[:M], DEC_EP_RELU, ln=ln)
+        assert torch.equal(y[:M].view(torch.int16), full[:M].view(torch.int16)), M
+        assert (y[M] == 7.0).all(), M
+
+
 @pytest.mark.parametrize("N,K,w8", [(1024, 1024, False), (1024, 4096, True), (1024, 4096, False)])
 @pytest.mark.parametrize("M", [1, 16, 24, 32, 37, 64])
 def test_dec_linear_fused_residual(N, K, w8, M, gpu):
