@@ -11,6 +11,7 @@
 #include "common.h"
 
 #include <string>
+#include <type_traits>
 
 namespace {
 
@@ -146,7 +147,9 @@ struct AttnShape {
   static constexpr int DP = D + 8;            // LDS row of K / R tiles (elements; 16-byte aligned, off bank stride)
   static constexpr int OB = D / 16;           // 16-dim blocks of the output
   static constexpr int VT = AT_KEYS + 4;      // LDS row of the transposed value tile
-  // key and value tiles double-buffered where three workgroups still fit a CU's 160 KB (one barrier per key tile)
+  // key and value tiles double-buffered where three workgroups still fit a CU's 160 KB (one barrier per key tile);
+  // head size 160 with two buffers, one workgroup a CU, was slower (bf16 block, 8 heads over 2250 rows 255 -> 275 us)
+  // and no faster where every workgroup has a CU to itself (one 376-frame clip 144 -> 147 us)
   static constexpr int NBUF = D <= 96 ? 2 : 1;
   static constexpr int K_ELEMS = AT_KEYS * DP, V_ELEMS = D * VT, R_ELEMS = AT_RING * DP, P_ELEMS = 4 * 16 * AT_PW;
   static constexpr int LDS_BYTES = 2 * (NBUF * (K_ELEMS + V_ELEMS) + R_ELEMS + P_ELEMS);
@@ -165,6 +168,7 @@ struct AttnArgs {
 };
 
 typedef short v4s __attribute__((ext_vector_type(4)));
+typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
 
 // 16 bytes at element offset off of a uniform base: a 32-bit byte offset from the base in scalar registers
 DEVI uint4 ld16(const uint16_t* base, uint32_t off) {
@@ -240,6 +244,93 @@ relpos_attention_kernel(const AttnArgs p) {
   const int HD = p.H * D, ld = 3 * HD;
   uint16_t* sPw = sP + w * 16 * AT_PW;
 
+  const uint16_t* kbase = p.qkv + (int64_t)start * ld + HD + h * D;
+  const uint16_t* vbase = kbase + HD;
+  const uint16_t* rbase = p.rk + h * D;
+  constexpr int CH = D / 8;  // 16-byte chunks per row
+  // a key tile's global data: keys j0 .. j0 + 31, their values, and the 32 table rows of distances
+  // q0 - j0 - 31 .. q0 - j0 (the tile reads distances up to q0 - j0 + 63; the previous tiles brought those). Loaded
+  // into registers one tile ahead, so the loads of tile j0 + 32 fly while tile j0 computes. The tile is KSL wave loads
+  // (64 chunks each) of keys, as many of table rows, and VSL pairs of wave loads of values, dealt to the four waves in
+  // that order, SL each: every wave issues the same loads with no branch between them, so no wait for an earlier load
+  // is needed among them (with loads under per-thread conditions the compiler put one there, a memory latency in each
+  // tile of every wave that fetched values). With the ring's first rows loaded in one go as well, head size 160 over
+  // one 376-frame clip of 8 heads went from 30.3 to 24.6 us and over 8 clips from 30.7 to 25.1; head size 80, with three
+  // workgroups a CU to cover such waits, from 31.7 to 31.1 over 8 clips of 375 frames. A load's chunk is (row id / CH, chunk id % CH) for keys and table rows;
+  // for values it is (key pair item % 16, chunk item / 16), so that the pair's 8 dims go to LDS as 8 dwords of the
+  // transposed tile with the lanes of a wave on distinct banks. 32-bit element offsets from uniform bases (a layer's
+  // qkv and table stay below 2^31 elements); keys past the sequence load its last key (their scores are masked and
+  // their probabilities exactly 0, the values finite, so no register is zeroed) and table rows are clamped to the
+  // table.
+  constexpr int VPAIRS = AT_KEYS / 2 * CH;                   // (key pair, chunk) items of values
+  constexpr int KSL = AT_KEYS * CH / 64, VSL = (VPAIRS + 63) / 64;
+  constexpr int SL = ((2 * KSL + 2 * VSL + 3) / 4 + 1) & ~1;  // loads per wave, even: a value pair stays in one wave
+  static_assert(AT_KEYS * CH % 64 == 0 && 2 * KSL % 2 == 0, "whole wave loads");
+  uint4 pre[SL];
+  int srow[SL], scol[SL];  // row in the tile and first element of this lane's chunk of each load
+  uint64_t sbase[SL];      // and, per wave, its source: address, row stride, last row, first row of tile 0
+  int sld[SL], shi[SL], sr0[SL], sdir[SL];
+#pragma unroll
+  for (int i = 0; i < SL; ++i) {
+    const int sl = w * SL + i, id = (sl < KSL ? sl : sl - KSL) * 64 + lane;
+    const int item = min((sl - 2 * KSL) / 2 * 64 + lane, VPAIRS - 1);
+    const bool r = sl >= KSL && sl < 2 * KSL, v = sl >= 2 * KSL;
+    srow[i] = v ? item % 16 * 2 + (i & 1) : id / CH;
+    scol[i] = v ? item / 16 * 8 : id % CH * 8;
+    const uint64_t ka = reinterpret_cast<uint64_t>(kbase), va = reinterpret_cast<uint64_t>(vbase);
+    sbase[i] = r ? reinterpret_cast<uint64_t>(rbase) : (v ? va : ka);
+    sld[i] = r ? HD : 3 * HD;
+    shi[i] = (r ? p.rel_rows : tile.y) - 1;
+    sr0[i] = r ? tile.z - (AT_KEYS - 1) + p.rel_off : 0;  // the tile's first new distance's row
+    sdir[i] = r ? -1 : 1;                                 // distances fall as keys advance
+  }
+  auto fetch = [&](int j0) {
+#pragma unroll
+    for (int i = 0; i < SL; ++i) {
+      const int row = min(max(sr0[i] + sdir[i] * j0 + srow[i], 0), shi[i]);
+      typedef const __attribute__((address_space(1))) char* gptr;
+      typedef const __attribute__((address_space(1))) uint4v* gvec;
+      const uint4v v = *(gvec)((gptr)sbase[i] + (((uint32_t)row * (uint32_t)sld[i] + (uint32_t)scol[i]) << 1));
+      pre[i] = make_uint4(v.x, v.y, v.z, v.w);
+    }
+  };
+  auto stash = [&](int j0, uint16_t* sK, uint16_t* sVt) {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the loads, a tile ago, on every path below
+    const int kofs = (int)(sK - lds), rofs = (int)(sR - lds);
+#pragma unroll
+    for (int i = 0; i < SL; i += 2) {
+      const int sl = w * SL + i;
+      if (sl < 2 * KSL) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const bool r = sl + k >= KSL;
+          const int row = ((r ? sr0[i + k] - j0 : 0) + srow[i + k]) & (AT_RING - 1);
+          *reinterpret_cast<uint4*>(lds + (r ? rofs : kofs) + row * S::DP + scol[i + k]) = pre[i + k];
+        }
+      } else if ((sl - 2 * KSL) / 2 * 64 + lane < VPAIRS) {
+        const uint32_t a[4] = {pre[i].x, pre[i].y, pre[i].z, pre[i].w};
+        const uint32_t b[4] = {pre[i + 1].x, pre[i + 1].y, pre[i + 1].z, pre[i + 1].w};
+        uint16_t* dst = sVt + scol[i] * S::VT + srow[i];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          *reinterpret_cast<uint32_t*>(dst + 2 * k * S::VT) = (a[k] & 0xffffu) | (b[k] << 16);
+          *reinterpret_cast<uint32_t*>(dst + (2 * k + 1) * S::VT) = (a[k] >> 16) | (b[k] & 0xffff0000u);
+        }
+      }
+    }
+  };
+  // the first tile also reads distances q0 + 1 .. q0 + 63: all their loads together, then into the ring (the last
+  // load's spare threads repeat the last chunk)
+  constexpr int NR = ((AT_Q - 1) * CH + 255) / 256;
+  uint4 ring[NR];
+#pragma unroll
+  for (int x = 0; x < NR; ++x) {
+    const int id = min(tid + x * 256, (AT_Q - 1) * CH - 1);
+    const int trow = min(max(q0 + 1 + id / CH + p.rel_off, 0), p.rel_rows - 1);
+    ring[x] = ld16(rbase, (uint32_t)trow * (uint32_t)HD + (uint32_t)(id % CH * 8));
+  }
+  fetch(0);
+
   // this lane's query plus either bias, as the B operand of both products
   const int qrow = q0 + 16 * w + iq;
   const bool qvalid = qrow < len;
@@ -248,92 +339,23 @@ relpos_attention_kernel(const AttnArgs p) {
   qu.load(qptr, p.bu + h * D, g, qvalid);
   qv.load(qptr, p.bv + h * D, g, qvalid);
 
+#pragma unroll
+  for (int x = 0; x < NR; ++x) {
+    const int id = min(tid + x * 256, (AT_Q - 1) * CH - 1);
+    const int d = q0 + 1 + id / CH;
+    *reinterpret_cast<uint4*>(sR + ((d + p.rel_off) & (AT_RING - 1)) * S::DP + id % CH * 8) = ring[x];
+  }
+
   v4f o[S::OB];
 #pragma unroll
   for (int i = 0; i < S::OB; ++i) o[i] = v4f{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;  // running maximum (natural units) and sum of this lane's query
 
-  const uint16_t* kbase = p.qkv + (int64_t)start * ld + HD + h * D;
-  const uint16_t* vbase = kbase + HD;
-  const uint16_t* rbase = p.rk + h * D;
-  constexpr int CH = D / 8;  // 16-byte chunks per row
-  // a key tile's global data: keys j0 .. j0 + 31, their values, and the 32 table rows of distances
-  // q0 - j0 - 31 .. q0 - j0 (the tile reads distances up to q0 - j0 + 63; the previous tiles brought those). Loaded
-  // into registers one tile ahead, so the loads of tile j0 + 32 fly while tile j0 computes. Chunk item x of a thread
-  // is (row id / CH, chunk id % CH) for keys and table rows; for values it is (key pair item % 16, chunk item / 16),
-  // so that the pair's 8 dims go to LDS as 8 dwords of the transposed tile with the lanes of a wave on distinct
-  // banks. 32-bit element offsets from uniform bases (a layer's qkv and table stay below 2^31 elements); keys past
-  // the sequence load its last key (their scores are masked and their probabilities exactly 0, the values finite, so
-  // no register is zeroed) and table rows are clamped to the table.
-  constexpr int NC = (AT_KEYS * CH + 255) / 256;      // key / table chunks per thread
-  constexpr int NV = (AT_KEYS / 2 * CH + 255) / 256;  // value chunk pairs per thread
-  uint4 pk[NC], pr[NC], pw[NV][2];
-#pragma unroll
-  for (int x = 0; x < NC; ++x) pk[x] = pr[x] = make_uint4(0, 0, 0, 0);  // once: the chunks past 32 rows
-#pragma unroll
-  for (int x = 0; x < NV; ++x) pw[x][0] = pw[x][1] = make_uint4(0, 0, 0, 0);
-  auto fetch = [&](int j0) {
-    const int d0 = q0 - j0 - (AT_KEYS - 1) + p.rel_off;  // table row of the tile's first new distance
-#pragma unroll
-    for (int x = 0; x < NC; ++x) {
-      const int id = tid + x * 256;
-      if (id < AT_KEYS * CH) {
-        const int r = id / CH, c = (id % CH) * 8, key = min(j0 + r, len - 1);
-        pk[x] = ld16(kbase, (uint32_t)key * (uint32_t)ld + (uint32_t)c);
-        const int trow = min(max(d0 + r, 0), p.rel_rows - 1);
-        pr[x] = ld16(rbase, (uint32_t)trow * (uint32_t)HD + (uint32_t)c);
-      }
-    }
-#pragma unroll
-    for (int x = 0; x < NV; ++x) {
-      const int item = tid + x * 256;
-      if (item < AT_KEYS / 2 * CH) {
-        const int rp = item % 16, c = (item / 16) * 8;
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-          const int key = min(j0 + 2 * rp + k, len - 1);
-          pw[x][k] = ld16(vbase, (uint32_t)key * (uint32_t)ld + (uint32_t)c);
-        }
-      }
-    }
-  };
-  auto stash = [&](int j0, uint16_t* sK, uint16_t* sVt) {
-#pragma unroll
-    for (int x = 0; x < NC; ++x) {
-      const int id = tid + x * 256;
-      if (id < AT_KEYS * CH) {
-        const int r = id / CH, c = (id % CH) * 8;
-        *reinterpret_cast<uint4*>(sK + r * S::DP + c) = pk[x];
-        const int d = q0 - j0 - (AT_KEYS - 1) + r;
-        *reinterpret_cast<uint4*>(sR + ((d + p.rel_off) & (AT_RING - 1)) * S::DP + c) = pr[x];
-      }
-    }
-#pragma unroll
-    for (int x = 0; x < NV; ++x) {
-      const int item = tid + x * 256;
-      if (item < AT_KEYS / 2 * CH) {
-        const int rp = item % 16, c = (item / 16) * 8;
-        const uint32_t a[4] = {pw[x][0].x, pw[x][0].y, pw[x][0].z, pw[x][0].w};
-        const uint32_t b[4] = {pw[x][1].x, pw[x][1].y, pw[x][1].z, pw[x][1].w};
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-          *reinterpret_cast<uint32_t*>(sVt + (c + 2 * k) * S::VT + 2 * rp) = (a[k] & 0xffffu) | (b[k] << 16);
-          *reinterpret_cast<uint32_t*>(sVt + (c + 2 * k + 1) * S::VT + 2 * rp) = (a[k] >> 16) | (b[k] & 0xffff0000u);
-        }
-      }
-    }
-  };
-  // the first tile also reads distances q0 + 1 .. q0 + 63, straight into the ring
-  for (int id = tid; id < (AT_Q - 1) * CH; id += 256) {
-    const int d = q0 + 1 + id / CH, c = (id % CH) * 8;
-    const int trow = min(max(d + p.rel_off, 0), p.rel_rows - 1);
-    *reinterpret_cast<uint4*>(sR + ((d + p.rel_off) & (AT_RING - 1)) * S::DP + c) =
-        *reinterpret_cast<const uint4*>(p.rk + (int64_t)trow * HD + h * D + c);
-  }
-
-  // one key tile from the given key and value buffers: scores, the online softmax and the value product
+  // one key tile from the given key and value buffers: scores, the online softmax and the value product; LAST: keys may
+  // lie past the sequence
   constexpr float L2E = 1.4426950408889634f;
-  auto key_tile = [&](int j0, const uint16_t* sK, const uint16_t* sVt) {
+  auto key_tile = [&](auto last, int j0, const uint16_t* sK, const uint16_t* sVt) {
+    constexpr bool LAST = decltype(last)::value;
     // position term of this wave's queries: distances dw0 + db, db < 48 (3 blocks of 16), its three products
     // interleaved per k step; then the content scores of keys kb * 16 + 4 g + e while those finish
     const int dw0 = q0 + 16 * w - j0 - (AT_KEYS - 1);
@@ -365,7 +387,8 @@ relpos_attention_kernel(const AttnArgs p) {
     // the 8 position scores of this lane, read together: key k = kb·16 + 4g + e sits at element
     // iq·(AT_PW + 1) + 31 - k of the wave's buffer, inside it for every key, so no read waits under the key mask.
     // Eight half-word reads from one base, written out so that the compiler neither fuses neighbours into misaligned
-    // wider reads nor moves each read under the mask, one after another.
+    // wider reads nor moves each read under the mask, one after another (no result may take the base's register: the
+    // reads after it use the base).
     float pos[8];
     {
       const uint32_t a = (uint32_t)reinterpret_cast<uintptr_t>(sPw + iq * AT_PW + iq + AT_KEYS - 1 - g * 4 - 19);
@@ -374,7 +397,8 @@ relpos_attention_kernel(const AttnArgs p) {
           "ds_read_u16 %0, %8 offset:38\n\tds_read_u16 %1, %8 offset:36\n\tds_read_u16 %2, %8 offset:34\n\t"
           "ds_read_u16 %3, %8 offset:32\n\tds_read_u16 %4, %8 offset:6\n\tds_read_u16 %5, %8 offset:4\n\t"
           "ds_read_u16 %6, %8 offset:2\n\tds_read_u16 %7, %8\n\ts_waitcnt lgkmcnt(0)"
-          : "=v"(r[0]), "=v"(r[1]), "=v"(r[2]), "=v"(r[3]), "=v"(r[4]), "=v"(r[5]), "=v"(r[6]), "=v"(r[7])
+          : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]), "=&v"(r[4]), "=&v"(r[5]), "=&v"(r[6]),
+            "=&v"(r[7])
           : "v"(a)
           : "memory");
 #pragma unroll
@@ -388,7 +412,7 @@ relpos_attention_kernel(const AttnArgs p) {
     for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
       for (int e = 0; e < 4; ++e) sv[kb * 4 + e] = __builtin_fmaf(s[kb][e], p.scale, pos[kb * 4 + e]);
-    if (j0 + AT_KEYS > len) {
+    if (LAST && j0 + AT_KEYS > len) {
 #pragma unroll
       for (int k = 0; k < 8; ++k) sv[k] = j0 + (k >> 2) * 16 + g * 4 + (k & 3) < len ? sv[k] : -INFINITY;
     }
@@ -422,29 +446,34 @@ relpos_attention_kernel(const AttnArgs p) {
     }
   };
 
-  fetch(0);
+  constexpr std::integral_constant<bool, false> full;
+  constexpr std::integral_constant<bool, true> last;
+  const int n_tiles = (len + AT_KEYS - 1) / AT_KEYS;
+  stash(0, sK0, sV0);
+  __syncthreads();
   if constexpr (S::NBUF == 2) {
     // tile t computes from buffer t & 1 while tile t + 1's data goes to the other one; the barrier after each tile
     // publishes the next tile and retires the reads of this one. The table rows tile t + 1 adds to the ring
     // (distances q0 - j0 - 63 .. q0 - j0 - 32) are not among the 96 that tile t reads (q0 - j0 - 31 .. q0 - j0 + 64),
     // modulo the ring's 128, so they are written while tile t computes
-    stash(0, sK0, sV0);
-    __syncthreads();
-    for (int j0 = 0, t = 0; j0 < len; j0 += AT_KEYS, ++t) {
-      const bool more = j0 + AT_KEYS < len;
-      if (more) fetch(j0 + AT_KEYS);
-      key_tile(j0, sK0 + (t & 1) * S::K_ELEMS, sV0 + (t & 1) * S::V_ELEMS);
-      if (more) stash(j0 + AT_KEYS, sK0 + ((t + 1) & 1) * S::K_ELEMS, sV0 + ((t + 1) & 1) * S::V_ELEMS);
+    int j0 = 0, b = 0;
+    for (int t = 1; t < n_tiles; ++t, j0 += AT_KEYS, b ^= 1) {
+      fetch(j0 + AT_KEYS);
+      key_tile(full, j0, sK0 + b * S::K_ELEMS, sV0 + b * S::V_ELEMS);
+      stash(j0 + AT_KEYS, sK0 + (b ^ 1) * S::K_ELEMS, sV0 + (b ^ 1) * S::V_ELEMS);
       __syncthreads();
     }
+    key_tile(last, j0, sK0 + b * S::K_ELEMS, sV0 + b * S::V_ELEMS);
   } else {
-    for (int j0 = 0; j0 < len; j0 += AT_KEYS) {
-      stash(j0, sK0, sV0);
-      __syncthreads();
-      if (j0 + AT_KEYS < len) fetch(j0 + AT_KEYS);
-      key_tile(j0, sK0, sV0);
+    int j0 = 0;
+    for (int t = 1; t < n_tiles; ++t, j0 += AT_KEYS) {
+      fetch(j0 + AT_KEYS);
+      key_tile(full, j0, sK0, sV0);
       __syncthreads();  // every wave is done with the key and value tiles
+      stash(j0 + AT_KEYS, sK0, sV0);
+      __syncthreads();
     }
+    key_tile(last, j0, sK0, sV0);
   }
 
   if (!qvalid) return;

@@ -126,6 +126,14 @@ def test_relpos_attention(gpu, H, D, lengths):
     _close_to_checker(_bits(out), want)
 
 
+@pytest.mark.parametrize("H,D", [(8, 160), (16, 80)])
+def test_relpos_attention_tile_edges(gpu, H, D):
+    """Each wave's share of a key tile's loads, and the last tile taken apart from the loop: lengths of one key more,
+    one less and exactly one, two, three and four tiles, all inside one batch whose neighbours hold other values. The
+    bar is the one the kernel has elsewhere (bf16 probabilities, sums in another order)."""
+    test_relpos_attention(gpu, H, D, [31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129])
+
+
 def test_relpos_attention_rejects_long_sequences(gpu):
     from kernels.fast_encoder import metadata
 
