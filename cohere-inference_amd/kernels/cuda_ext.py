@@ -217,7 +217,8 @@ class _Ext:
 
     def sub_conv0_dw_pw(self, feats, mel_len, rows, w0, b0, w2, b2, wp, bp, out):
         """sub_conv0_dw, then the stem's pointwise convolution of its output with wp (256, 256) and bp (256) bf16 and
-        ReLU (gemm with EPI_CONV_RELU), in one launch: out (n, 32, 256); the same bits as the two calls."""
+        ReLU (gemm with EPI_CONV_RELU), in one launch: out (n, 32, 256). conv0's fp32 sums are in another order
+        than the two calls', so a rounding moves by one bf16 step now and then."""
         _check(feats.is_contiguous() and feats.dim() == 3 and feats.shape[2] == 128 and
                feats.dtype == torch.bfloat16 and w0.shape[0] == 256 and rows.dtype == torch.int32 and
                rows.is_contiguous() and mel_len.dtype == torch.int32 and
@@ -232,7 +233,8 @@ class _Ext:
                    _ptr(b0), _ptr(w2), _ptr(b2), _ptr(wp), _ptr(bp), _ptr(out), _stream())
 
     def sub_dw_pw(self, x, in_start, in_len, rows, w, b, wp, bp, out):
-        """sub_dw on x (sum T_in, 32, 256), then the stem's pointwise convolution as sub_conv0_dw_pw: out (n, 16, 256)."""
+        """sub_dw on x (sum T_in, 32, 256), then the stem's pointwise convolution as sub_conv0_dw_pw: out (n, 16, 256);
+        the same bits as the two calls."""
         n = rows.shape[0]
         _check(x.is_contiguous() and x.dim() == 3 and tuple(x.shape[1:]) == (32, 256) and
                x.dtype == torch.bfloat16 and rows.dtype == torch.int32 and rows.is_contiguous() and
