@@ -431,29 +431,30 @@ DEVI void pointwise(char* tile, const uint16_t* __restrict__ w, const uint16_t* 
 }
 
 // The same two convolutions and the pointwise one that follows, for C = 256, SUB_T output rows (sequence, t2) per
-// workgroup. On the vector units a conv0 value takes 9 multiply-adds and 7 more instructions, and that issue is all of
-// the kernel above (129 us for 8 pieces of 30 s; with conv0 rows shared between output rows and the pointwise
-// convolution behind it 153). So conv0 runs on the matrix cores: a bf16 mel value and a third of a weight's bits are
-// exact factors, and a weight is the exact sum of three bf16 values (its leading, middle and last 8 bits), so one
-// K = 32 instruction holds the 27 products of a 3 x 3 patch and adds them in fp32 (stem of 8 pieces of 30 s against 64
-// bits: 4.8e-3 either way). Everything after the sum is as above, in the same order. 8 pieces of 30 s: 113 us for what
-// the two launches took 180; what is left is the vector work after the sums (about 60 us) and the phases' latencies.
-//  * A operand: the patches of one conv0 row, 64 positions x 32 K values, gathered in LDS one row ahead of their use
-//    (K index 9 q + tap: tap value for weight part q). Row m of block pb is position 16 (m / 4) + 4 pb + m % 4, so a
-//    lane holds 16 consecutive positions of a channel and the depthwise taps need one value from another lane.
+// workgroup; the same bits as the two launches. On the vector units a conv0 value takes 9 multiply-adds and 7 more
+// instructions, and that issue is all of the kernel above (129 us for 8 pieces of 30 s; with conv0 rows shared between
+// output rows and the pointwise convolution behind it 153). So conv0's multiply-adds run on the matrix cores, one
+// instruction a tap: with K = 1 in fp32 it adds each position's product to the sum before it with one rounding, the
+// fma of the chain above. (All taps in one bf16 instruction, a weight as three exact bf16 parts, sums them in another
+// order, with 1.4 times the rounding error where mel values span many powers of two.) 8 pieces of 30 s: 115 us
+// for what the two launches take 169; what is left is the vector work after the sums (about 60 us).
+//  * The matrix instruction's four blocks of 16 rows are the 64 positions of a conv0 row: row m of block pb is position
+//    16 (m / 4) + 4 pb + m % 4, so a lane holds 16 consecutive positions of a channel and the depthwise taps need one
+//    value from another lane.
 //  * Where the next row of the list is t2 + 1 of the same sequence (the stem's lists), conv0 row 2 t2 + 1 is computed
 //    once and added to both rows' sums.
 //  * The rows stay in LDS as the pointwise convolution's operand; only its output is written.
 constexpr int SUB_T = 4, SUB_W = 8, SUB_J = 16 / SUB_W;  // output rows, waves, 16-channel blocks of a wave
-constexpr int MEL_LD = MELS + 8, PATCH = 64 * 64;         // patch bytes of a conv0 row
+constexpr int MEL_LD = MELS + 8;
+typedef float v16f __attribute__((ext_vector_type(16)));
 __global__ void __launch_bounds__(SUB_W * 64) __attribute__((amdgpu_waves_per_eu(4))) sub_conv0_dw_pw_kernel(
     const uint16_t* __restrict__ feats, int64_t ld_seq, const int* __restrict__ mel_len, const int* __restrict__ rows,
     int n_rows, const float* __restrict__ w0, const float* __restrict__ b0, const float* __restrict__ w2,
     const float* __restrict__ b2, const uint16_t* __restrict__ wp, const uint16_t* __restrict__ bp,
     uint16_t* __restrict__ out) {
   __shared__ __attribute__((aligned(16))) char tile[SUB_T * SUB_F2 * 2 * PW_C];
-  __shared__ __attribute__((aligned(16))) char patch[2][PATCH];
-  __shared__ uint16_t mel[SUB_T][7][MEL_LD];  // mel rows 4 t2 - 3 .. 4 t2 + 3, column c at c + 1, zeros outside
+  // mel rows 4 t2 - 3 .. 4 t2 + 3, column c at c + 1, zeros outside
+  __shared__ __attribute__((aligned(8))) uint16_t mel[SUB_T][7][MEL_LD];
   const int tid = threadIdx.x, lane = lane_id(), wave = wave_id(), c16 = lane & 15, h = lane >> 4;
   const int i0 = blockIdx.x * SUB_T, nt = min(SUB_T, n_rows - i0);
   // one thread per pair of columns of the seven rows, every load unguarded (a row outside the sequence loads row 0)
@@ -467,77 +468,44 @@ __global__ void __launch_bounds__(SUB_W * 64) __attribute__((amdgpu_waves_per_eu
     const u32_any v = *reinterpret_cast<const u32_any*>(feats + (int64_t)seq * ld_seq + (in ? (int64_t)r * MELS : 0) + mc);
     mv[k] = in ? (uint32_t)v : 0u;
   }
-  // this lane's channels (wave * SUB_J + j) * 16 + c16: conv0 weights as the B operand (K 8 h .. 8 h + 7), depthwise taps
-  v8bf wf[SUB_J];
-  float kd[SUB_J][9], bias0[SUB_J], bias2[SUB_J];
+  // this lane's channels (wave * SUB_J + j) * 16 + c16: conv0 weights (the B operand, the same in all four blocks) and
+  // depthwise taps
+  float wf[SUB_J][9], kd[SUB_J][9], bias0[SUB_J], bias2[SUB_J];
 #pragma unroll
   for (int j = 0; j < SUB_J; ++j) {
     const int c = (wave * SUB_J + j) * 16 + c16;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int kk = 8 * h + e, q = kk / 9;
-      float w = w0[c * 9 + kk % 9];
-      const bool finite = __builtin_isfinite(w);
-      // part q of the weight: the 8 leading bits of what the parts before it leave (by truncation: each part exact); an
-      // infinity or NaN is its first part
-      float part = 0.f;
-#pragma unroll
-      for (int i = 0; i < 3; ++i) {
-        part = i <= q ? __uint_as_float(__float_as_uint(w) & 0xffff0000u) : part;
-        w = i < q ? w - part : w;
-      }
-      wf[j][e] = __builtin_bit_cast(__bf16, (uint16_t)(__float_as_uint(kk < 27 && (finite || q == 0) ? part : 0.f) >> 16));
+    for (int i = 0; i < 9; ++i) {
+      wf[j][i] = w0[c * 9 + i];
+      kd[j][i] = w2[c * 9 + i];
     }
-#pragma unroll
-    for (int i = 0; i < 9; ++i) kd[j][i] = w2[c * 9 + i];
     bias0[j] = b0[c];
     bias2[j] = b2[c];
   }
-  // the patch values this thread gathers: position f1 of A row tid / 8, K values 4 (tid % 8) .. + 3
-  static_assert(SUB_W == 8, "one thread per 4 K values of a position");
-  const int pm = tid >> 3, pq = tid & 7, f1 = 16 * ((pm & 15) >> 2) + 4 * (pm >> 4) + (pm & 3);
-  // from the patch's first mel value; the 5 spare K values are zero, and so is an infinity or NaN beside the second and
-  // third weight parts (which may be zero)
-  int off[4];
-  uint32_t drop[4];  // exponent bits whose presence in full makes the value zero
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    const int kk = 4 * pq + e, tap = kk % 9;
-    off[e] = kk < 27 ? tap / 3 * MEL_LD + tap % 3 : 0;
-    drop[e] = kk < 9 ? 0x10000u : kk < 27 ? 0x7f80u : 0u;
-  }
-  auto gather = [&](int b, int k, int r) {  // conv0 row of tap row r of output row k
-    const uint16_t* src = &mel[k][2 * r][2 * f1];
-    uint32_t v[2];
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      uint32_t lo = src[off[2 * e]], hi = src[off[2 * e + 1]];
-      lo = (lo & drop[2 * e]) == drop[2 * e] ? 0u : lo;
-      hi = (hi & drop[2 * e + 1]) == drop[2 * e + 1] ? 0u : hi;
-      v[e] = lo | hi << 16;
-    }
-    *reinterpret_cast<uint2*>(patch[b] + pm * 64 + (((pq >> 1) ^ ((pm >> 2) & 3)) << 4) + (pq & 1) * 8) =
-        make_uint2(v[0], v[1]);
-  };
+  const int f1 = 16 * (c16 >> 2) + 4 * h + (c16 & 3);  // this lane's position as A operand: row c16 of block h
   float acc[SUB_J][8], acc2[SUB_J][8];  // depthwise sums of this lane's channels at f2 = 8 h + o, this output row's and the next's
-  // one conv0 row added as tap row r (and, both, to the next output row as tap row 0)
-  auto conv_row = [&](int b, int r, bool both) {
-    v8bf a[4];
+  // the conv0 row of output row k's tap row r, added as that tap row (and, both, to the next output row as tap row 0)
+  auto conv_row = [&](int k, int r, bool both) {
+    float x[9];
 #pragma unroll
-    for (int pb = 0; pb < 4; ++pb)
-      a[pb] = *reinterpret_cast<const v8bf*>(patch[b] + (pb * 16 + c16) * 64 + ((h ^ (c16 >> 2)) << 4));
+    for (int i = 0; i < 3; ++i) {
+      const uint32_t* m = reinterpret_cast<const uint32_t*>(&mel[k][2 * r + i][2 * f1]);
+      const uint32_t lo = m[0], hi = m[1];
+      x[3 * i] = __uint_as_float(lo << 16);
+      x[3 * i + 1] = __uint_as_float(lo & 0xffff0000u);
+      x[3 * i + 2] = __uint_as_float(hi << 16);
+    }
 #pragma unroll
     for (int j = 0; j < SUB_J; ++j) {
+      v16f d = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < 9; ++i) d = __builtin_amdgcn_mfma_f32_16x16x1f32(x[i], wf[j][i], d, 0, 0, 0);
       float v[16];
 #pragma unroll
-      for (int pb = 0; pb < 4; ++pb) {
-        const v4f d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[pb], wf[j], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-        for (int q = 0; q < 2; ++q) {
-          const uint32_t u = pack_bf2(d[2 * q], d[2 * q + 1]);  // rounded, then the bias, ReLU and the second rounding
-          v[4 * pb + 2 * q] = round_bf_valu(fmaxf(__uint_as_float(u << 16) + bias0[j], 0.f));
-          v[4 * pb + 2 * q + 1] = round_bf_valu(fmaxf(__uint_as_float(u & 0xffff0000u) + bias0[j], 0.f));
-        }
+      for (int q = 0; q < 16; q += 2) {
+        const uint32_t u = pack_bf2(d[q], d[q + 1]);  // rounded, then the bias, ReLU and the second rounding
+        v[q] = round_bf_valu(fmaxf(__uint_as_float(u << 16) + bias0[j], 0.f));
+        v[q + 1] = round_bf_valu(fmaxf(__uint_as_float(u & 0xffff0000u) + bias0[j], 0.f));
       }
       // position 16 h - 1: the last one of the lane 16 below (none for h = 0)
       const float left = __shfl(v[15], (lane - 16) & 63, 64);
@@ -547,8 +515,8 @@ __global__ void __launch_bounds__(SUB_W * 64) __attribute__((amdgpu_waves_per_eu
 #pragma unroll
         for (int o = 0; o < 8; ++o) {
           if (o == 0) {
-            const float x = __builtin_fmaf(k0, left, s[0]);
-            s[0] = h > 0 ? x : s[0];
+            const float y = __builtin_fmaf(k0, left, s[0]);
+            s[0] = h > 0 ? y : s[0];
           } else {
             s[o] = __builtin_fmaf(k0, v[2 * o - 1], s[o]);
           }
@@ -582,23 +550,15 @@ __global__ void __launch_bounds__(SUB_W * 64) __attribute__((amdgpu_waves_per_eu
     mel[row / 7][row % 7][e == 0 ? 0 : MELS + e] = 0;
   }
   __syncthreads();  // mel rows
-  gather(0, 0, 0);
-  __syncthreads();
   bool carried = false;  // acc holds this row's tap row 0
-  int b = 0;
   clear(acc);
   for (int k = 0; k < nt; ++k) {
     const int seq = rows[2 * (i0 + k)], t2 = rows[2 * (i0 + k) + 1], T1 = (mel_len[seq] - 1) / 2 + 1;
     const bool next = follows(k);
     for (int r = carried ? 1 : 0; r < 3; ++r) {
-      // gather the row that comes after this one: the next tap row, or the next output row's first
-      if (r < 2) gather(b ^ 1, k, r + 1);
-      else if (k + 1 < nt) gather(b ^ 1, k + 1, next ? 1 : 0);
       const int t1 = 2 * t2 - 1 + r;
       if (r == 2 && next) clear(acc2);
-      if (t1 >= 0 && t1 < T1) conv_row(b, r, r == 2 && next);
-      __syncthreads();  // the next patches are written, these are read
-      b ^= 1;
+      if (t1 >= 0 && t1 < T1) conv_row(k, r, r == 2 && next);
     }
 #pragma unroll
     for (int j = 0; j < SUB_J; ++j)

@@ -217,8 +217,7 @@ class _Ext:
 
     def sub_conv0_dw_pw(self, feats, mel_len, rows, w0, b0, w2, b2, wp, bp, out):
         """sub_conv0_dw, then the stem's pointwise convolution of its output with wp (256, 256) and bp (256) bf16 and
-        ReLU (gemm with EPI_CONV_RELU), in one launch: out (n, 32, 256). conv0's fp32 sums are in another order
-        than the two calls', so a rounding moves by one bf16 step now and then."""
+        ReLU (gemm with EPI_CONV_RELU), in one launch: out (n, 32, 256); the same bits as the two calls."""
         _check(feats.is_contiguous() and feats.dim() == 3 and feats.shape[2] == 128 and
                feats.dtype == torch.bfloat16 and w0.shape[0] == 256 and rows.dtype == torch.int32 and
                rows.is_contiguous() and mel_len.dtype == torch.int32 and

@@ -338,8 +338,8 @@ int cohere_sub_dw(const uint16_t* x, const int32_t* in_start, const int32_t* in_
 
 /* sub_conv0_dw with 256 channels, then the pointwise convolution that follows it in the stem (reference
  * kernels/fast_encoder.py:193-199: gemm with CONV_RELU): wp bf16 [256, 256] (output channel, input channel), bp bf16
- * [256]; out bf16 [n_rows, 32, 256] = relu(bf16(pointwise sum) + bp). conv0's fp32 sums are in another order than in
- * the two calls: a rounding moves by one bf16 step now and then. 16-byte aligned wp and out, 8-byte aligned bp. */
+ * [256]; out bf16 [n_rows, 32, 256] = relu(bf16(pointwise sum) + bp). The same bits as the two calls. 16-byte aligned
+ * wp and out, 8-byte aligned bp. */
 int cohere_sub_conv0_dw_pw(const uint16_t* feats, int64_t ld_seq, const int32_t* mel_len, const int32_t* rows,
                            int64_t n_rows, const float* w0, const float* b0, const float* w2, const float* b2,
                            const uint16_t* wp, const uint16_t* bp, uint16_t* out, void* stream);
