@@ -21,7 +21,7 @@ bool tiles_bf16(int tile, const GemmArgs& p, hipStream_t s) {
   }
 }
 
-// the tiles of whole 128-column vectors
+// the tiles of kv_tile
 template <int EPI>
 bool tiles_kv(int tile, const GemmArgs& p, hipStream_t s) {
   switch (tile) {

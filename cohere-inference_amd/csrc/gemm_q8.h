@@ -888,6 +888,8 @@ int ref_config_group(int cfg);
 constexpr bool bf16_tile(int tile) {
   return tile == 0 || tile == 3 || tile == 6 || tile == 7 || tile == 8 || tile == 9 || tile == 15 || tile == 17;
 }
+// those of them with the cache epilogues (EPI_KV, EPI_KV8): whole 128-column vectors
+constexpr bool kv_tile(int tile) { return tile == 3 || tile == 6 || tile == 9 || tile == 15 || tile == 17; }
 bool launch_gemm_bf16(int tile, int epi, const GemmArgs& p, hipStream_t s);
 
 }  // namespace cohere_gemm

@@ -51,7 +51,7 @@ int choose_tile(const GemmArgs& p, bool grouped, bool bf = false) {
   auto fits = [&](int id) {
     const TileInfo& t = TILES[id];
     if (bf && !bf16_tile(id)) return false;
-    if ((p.epi == EPI_KV || p.epi == EPI_KV8) && (t.bn % 128 || id == 8)) return false;
+    if ((p.epi == EPI_KV || p.epi == EPI_KV8) && !kv_tile(id)) return false;
     if (p.N % t.bn) return false;
     if (grouped && !t.grouped_ok) return false;
     if (p.epi == EPI_SILU_Q8 && t.bn % p.qgroup) return false;

@@ -398,8 +398,8 @@ def test_decoder_built_behind_queued_work(gpu):
 @pytest.mark.parametrize("q8", [True, False])
 @pytest.mark.parametrize("rows,L,H", [(1, 1, 1), (70, 2, 3), (400, 3, 8), (1500, 8, 8)])
 def test_gemm_kv_equals_gemm_then_scatter(gpu, rows, L, H, q8):
-    """The projections with the caches' layout as their epilogue against the GEMM and the scatter launched in turn, from
-    the smallest tile to the largest: every byte of the caches and scales, rows in any slot order."""
+    """The projections with the caches' layout as their epilogue against the GEMM and the scatter launched in turn:
+    every byte of the caches and scales, rows in any slot order."""
     g = torch.Generator().manual_seed(rows + L + H)
     S, T, K, N = 5, 500, 96, L * 2 * H * 128
     a = torch.randn(rows, K, generator=g).to(torch.bfloat16).to(gpu)
@@ -417,3 +417,33 @@ def test_gemm_kv_equals_gemm_then_scatter(gpu, rows, L, H, q8):
         _ext().gemm_kv(a, w, bias, slot_of, frame_of, *got)
         for x, y in zip(got, want):
             assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("q8", [True, False])
+@pytest.mark.parametrize("rows,L,H,K", [(300, 1, 2, 1056), (750, 8, 8, 1024)])
+def test_gemm_kv_at_every_tile(gpu, rows, L, H, K, q8):
+    """Every forced tile, those without a cache epilogue among them (the choice by shape then stands): the same bytes as
+    the GEMM and the scatter, over more K stages than a tile's ring holds (1056: and a half one) and rows that fill no
+    tile."""
+    g = torch.Generator().manual_seed(rows + K)
+    S, T, N = 3, 300, L * 2 * H * 128
+    a = torch.randn(rows, K, generator=g).to(torch.bfloat16).to(gpu)
+    w = (0.1 * torch.randn(N, K, generator=g)).to(torch.bfloat16).to(gpu)
+    bias = torch.randn(N, generator=g).to(torch.bfloat16).to(gpu)
+    where = torch.randperm(S * T, generator=g)[:rows]
+    slot_of, frame_of = (where // T).to(torch.int32).to(gpu), (where % T).to(torch.int32).to(gpu)
+    new = lambda: ([torch.zeros(L, S, H, T, 128, device=gpu, dtype=torch.int8 if q8 else torch.bfloat16)  # noqa: E731
+                    for _ in range(2)] + ([torch.zeros(L, S, H, T, device=gpu) for _ in range(2)] if q8 else []))
+    kv, want = torch.empty(rows, N, dtype=torch.bfloat16, device=gpu), new()
+    _ext().gemm(a, w, bias, kv, 0, None, 1.0, 8)
+    (_ext().dec_scatter_kv_q8 if q8 else _ext().dec_scatter_kv)(kv, slot_of, frame_of, *want)
+    try:
+        for tile in range(-1, _ext().set_gemm_tile(-1)):
+            _ext().set_gemm_tile(tile)
+            print(f"gemm_kv tile {tile}", flush=True)
+            got = new()
+            _ext().gemm_kv(a, w, bias, slot_of, frame_of, *got)
+            for x, y in zip(got, want):
+                assert torch.equal(x, y), tile
+    finally:
+        _ext().set_gemm_tile(-1)
