@@ -24,25 +24,33 @@ int num_cus() {
   return n;
 }
 
-// The time of a round of workgroups, one per CU (64x64 tiles: two, the second costing a quarter more), on each tile, in
-// microseconds: c per 128-byte K stage, f for the launch, the first stage and the epilogue, q8 for SILU_Q8's. Fitted
-// to graph replays of the encoder's linears at 376, 1892, 3000 and 8416 rows (K 1280 and 5120) and the bf16 stem, cross-
-// attention and layer shapes; the model is within 10 % of most of them. Against the largest tile that gives 64 % of
-// the CUs a workgroup (the former rule): bf16 1892 x 1280 x 5120 62.2 -> 39.1 us, 1892 x 5120 x 1280 SILU 48.3 -> 39.7,
-// 1892 x 1280 x 1280 21.4 -> 13.9, 3000 x 1024 x 1280 15.0 -> 12.6; int8 3000 x 1280 x 1280 12.2 -> 9.5, grouped 1892 x
-// 1280 x 5120 42.7 -> 28.3.
+// The time of a round of workgroups, one per CU, on each tile, in microseconds: c per 128-byte K stage, f for the launch,
+// the first stage and the epilogue, q8 for SILU_Q8's. 64x64 tiles (per_cu 2): two share a CU, each stage then taking
+// 1.3 times as long, and what is more than that counts by half rounds. (As whole rounds of two with one workgroup's
+// time, 7000 grouped rows x 1280 x 5120 took 64x64 tiles, 110 us, where 128x128 ones take 83.)
+// Fitted to graph replays of the encoder's linears at 376, 1892, 3000 and 8416 rows (K 1280 and 5120) and the bf16 stem,
+// cross-attention and layer shapes. Every tile timed for 18 linears (int8, 2:4, grouped, bf16) at 32 row counts from 6 to
+// 9024: the choice is within 4 % of the fastest tile at 549 of 561 points (the rest are bf16, the worst 1280 x 1280 over
+// 7000 rows and more, 14 %), and nowhere slower than the former rule's beyond the noise of 2 %. Against that, the largest
+// tile that gives 64 % of the CUs a workgroup (the former rule): bf16 1892 x 1280 x 5120 62.2 -> 39.1 us, 1892 x 5120 x
+// 1280 SILU 48.3 -> 39.7, 1892 x 1280 x 1280 21.4 -> 13.9, 3000 x 1024 x 1280 15.0 -> 12.6; int8 3000 x 1280 x 1280 12.2
+// -> 9.5, grouped 1892 x 1280 x 5120 42.7 -> 28.3.
 struct TileCost {
   int id;
   int per_cu;
   double c, f, q8;
 };
-constexpr TileCost DENSE_COST[] = {{6, 1, 1.28, 10.9, 8.0}, {15, 1, 1.335, 10.0, 6.2}, {8, 1, .695, 7.5, 3.0},
+constexpr TileCost BF16_COST[] = {{6, 1, 1.28, 10.9, 0.0}, {15, 1, 1.335, 10.0, 0.0}, {8, 1, .695, 7.5, 0.0},
+                                  {9, 1, .69, 6.6, 0.0},   {17, 1, .42, 4.5, 0.0},    {3, 1, .353, 3.3, 0.0},
+                                  {7, 2, .265, 3.0, 0.0}};
+constexpr TileCost DENSE_COST[] = {{6, 1, 1.28, 10.9, 8.0}, {15, 1, 1.285, 10.5, 6.2}, {8, 1, .695, 7.5, 3.0},
                                    {9, 1, .69, 6.6, 3.0},   {17, 1, .42, 4.5, 2.0},    {4, 1, .6, 4.0, 3.3},
-                                   {3, 1, .353, 3.3, 2.0},  {5, 1, .27, 3.1, 2.0},     {7, 2, .265, 3.0, 2.0}};
+                                   {3, 1, .335, 3.3, 2.0},  {5, 1, .27, 3.1, 2.0},     {7, 2, .265, 3.0, 2.0}};
 // 2:4 weights; 10 reads stage-tiled records (row-major ones take 15)
 constexpr TileCost SPARSE_COST[] = {{10, 1, 1.03, 11.2, 7.0}, {15, 1, 1.25, 11.0, 7.0}, {8, 1, .58, 6.2, 3.5},
-                                    {9, 1, .52, 6.7, 3.5},    {17, 1, .47, 2.6, 2.0},   {0, 1, .437, 3.6, 2.0}, {4, 1, .447, 3.4, 4.1},
-                                    {3, 1, .35, 3.3, 2.0},    {5, 1, .27, 3.1, 2.0},    {7, 2, .25, 3.0, 2.0}};
+                                    {9, 1, .52, 6.7, 3.5},    {17, 1, .47, 2.6, 2.0},   {0, 1, .437, 3.6, 2.0},
+                                    {4, 1, .447, 3.4, 4.1},   {3, 1, .315, 3.3, 2.0},   {5, 1, .27, 3.1, 2.0},
+                                    {7, 2, .25, 3.0, 2.0}};
 // grouped scales (each group's fold is most of a stage); the larger 8-wave tiles spill
 constexpr TileCost GROUPED_COST[] = {{17, 1, .62, 3.6, 2.0}, {4, 1, .75, 3.5, 3.3},  {3, 1, .47, 3.4, 2.0},
                                      {5, 1, .35, 3.1, 2.0},  {7, 2, .34, 3.0, 2.0}};
@@ -58,26 +66,25 @@ int choose_tile(const GemmArgs& p, bool grouped, bool bf = false) {
     return true;
   };
   if (g_tile_override >= 0 && g_tile_override < N_TILES && fits(g_tile_override)) return g_tile_override;
-  // the tile whose model time is least: rounds of workgroups over the CUs, each (c per 128-byte K stage + f)
+  // the tile whose model time is least
   const double stages = p.K / 128.0;
   const int64_t cus = num_cus();
   int best = -1;
   double least = 0.0;
-  const TileCost* table = grouped ? GROUPED_COST : p.E ? SPARSE_COST : DENSE_COST;
-  const size_t n_costs = grouped  ? sizeof(GROUPED_COST) / sizeof(TileCost)
-                         : p.E    ? sizeof(SPARSE_COST) / sizeof(TileCost)
-                                  : sizeof(DENSE_COST) / sizeof(TileCost);
-  for (size_t k = 0; k < n_costs; ++k) {
-    const TileCost& t = table[k];
-    if (!fits(t.id) || (p.E && !p.tiled && t.id == 10)) continue;
-    const int64_t n = (int64_t)((p.M + TILES[t.id].bm - 1) / TILES[t.id].bm) * (p.N / TILES[t.id].bn);
-    const double rounds = t.per_cu == 1  ? (double)((n + cus - 1) / cus)
-                          : n <= cus     ? 1.0
-                          : n <= 2 * cus ? 1.25
-                                         : (double)((n + 2 * cus - 1) / (2 * cus));
-    const double us = rounds * (t.c * stages + t.f + (p.epi == EPI_SILU_Q8 ? t.q8 : 0.0));
-    if (best < 0 || us < least) best = t.id, least = us;
-  }
+  auto consider = [&](const auto& table) {
+    for (const TileCost& t : table) {
+      if (!fits(t.id) || (p.E && !p.tiled && t.id == 10)) continue;
+      const int64_t n = (int64_t)((p.M + TILES[t.id].bm - 1) / TILES[t.id].bm) * (p.N / TILES[t.id].bn);
+      const double rounds = (double)((n + cus - 1) / cus), once = t.f + (p.epi == EPI_SILU_Q8 ? t.q8 : 0.0);
+      const double us = t.per_cu == 1 || n <= cus ? rounds * (t.c * stages + once)
+                                                  : rounds / 2 * (1.3 * t.c * stages + once);
+      if (best < 0 || us < least) best = t.id, least = us;
+    }
+  };
+  if (grouped) consider(GROUPED_COST);
+  else if (p.E) consider(SPARSE_COST);
+  else if (bf) consider(BF16_COST);
+  else consider(DENSE_COST);
   return best;
 }
 
@@ -158,6 +165,17 @@ extern "C" int cohere_set_gemm_tile(int32_t tile) {
   }
   g_tile_override = tile;
   return N_TILES;
+}
+
+extern "C" int cohere_gemm_tile(int32_t kind, int32_t epi, int64_t M, int64_t N, int64_t K, int64_t group) {
+  if (kind < 0 || kind > 4 || M <= 0 || N <= 0 || K <= 0 || M >= (1LL << 31) || N >= (1LL << 31) || K >= (1LL << 30) ||
+      N % 64)
+    return -1;
+  const bool bf = kind >= 3;
+  GemmArgs p{};
+  p.M = (int)M; p.N = (int)N; p.K = (int)(bf ? 2 * K : K); p.epi = kind == 4 ? EPI_KV : epi; p.qgroup = 256;
+  p.E = kind == 1 || kind == 2 ? reinterpret_cast<const int32_t*>(&p) : nullptr; p.tiled = kind == 2;
+  return choose_tile(p, !bf && group < K, bf);
 }
 
 extern "C" int cohere_gemm_i8(const int8_t* a, int64_t lda, const float* sa, int64_t ldsa, int64_t group,

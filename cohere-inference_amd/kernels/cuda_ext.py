@@ -39,7 +39,7 @@ EXPORTS = ("cohere_gemm_i8", "cohere_gemm_sp", "cohere_quantize_rows", "cohere_l
            "cohere_logmel_features", "cohere_sub_conv0_dw", "cohere_sub_dw", "cohere_encoder_branch_workspace_bytes",
            "cohere_encoder_layers_noalloc", "cohere_dec_linear_fused", "cohere_dec_pick_embed",
            "cohere_gemm_sp_tiled", "cohere_pack_24_tiled_bytes", "cohere_pack_24_tiled", "cohere_sub_conv0_dw_pw",
-           "cohere_sub_dw_pw", "cohere_gemm_kv", "cohere_gemm_kv_q8")
+           "cohere_sub_dw_pw", "cohere_gemm_kv", "cohere_gemm_kv_q8", "cohere_gemm_tile")
 
 
 def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
@@ -60,6 +60,7 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
         "cohere_linear_bf16": [P, I64, P, P, P, I64, I32, I64, I64, I64, P],
         "cohere_dec_linear_fused": [P, I64, P, P, F, P, P, P, P, I64, I32, I64, I64, I64, P],
         "cohere_set_gemm_tile": [I32],
+        "cohere_gemm_tile": [I32, I32, I64, I64, I64, I64],
         "cohere_set_skinny_shape": [I32, I32],
         "cohere_layernorm": [P, I64, P, P, F, P, P, F, P, I64, I64, I64, P],
         "cohere_dwconv_bn_silu": [P, P, P, P, P, P, P, P, I64, I64, I64, P],
@@ -138,6 +139,10 @@ class _Ext:
     def set_gemm_tile(self, tile: int) -> int:
         """Tuning hook: force a gfx950 GEMM tile (-1 = automatic). Results never depend on it."""
         return self._lib.cohere_set_gemm_tile(int(tile))
+
+    def gemm_tile(self, kind: int, epi: int, M: int, N: int, K: int, group: int) -> int:
+        """Tuning hook: the tile a product of these sizes runs on (kind 0 int8, 1 2:4, 2 2:4 tiled, 3 bf16, 4 caches)."""
+        return self._lib.cohere_gemm_tile(kind, epi, M, N, K, group)
 
     def set_skinny_shape(self, strips: int, waves: int) -> None:
         """Tuning hook: force the skinny projections' workgroup shape (strips <= 0 = automatic)."""

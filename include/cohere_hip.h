@@ -361,6 +361,11 @@ const char* cohere_version(void);
  * Used by bench.py's sweeps; results never depend on it. Returns the number of tiles available. */
 int cohere_set_gemm_tile(int32_t tile);
 
+/* Tuning hook (no counterpart in the reference): the tile that a product of these sizes runs on, without launching it
+ * (few int8 rows may take the few-row kernel instead); -1 where none fits. kind: 0 int8 weights, 1 2:4 row-major, 2 2:4
+ * stage-tiled, 3 bf16, 4 bf16 into the cross-attention caches; group < K: scales per row and group. */
+int cohere_gemm_tile(int32_t kind, int32_t epi, int64_t M, int64_t N, int64_t K, int64_t group);
+
 /* Tuning hook (no counterpart in the reference): force the skinny projections' workgroup shape -- strips of 16
  * channels per workgroup (1, 2, 4) and waves per workgroup (4, 8, 16); strips <= 0 restores the automatic choice.
  * Results never depend on it. */

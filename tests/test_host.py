@@ -176,3 +176,43 @@ def test_pack_24_tiled_matches_c_abi_and_round_trips():
                 stored = rec[1024 + 16 * r:1040 + 16 * r].view(np.int32)
                 back_e[rb * 16 + r, kt * 4:kt * 4 + 4] = stored[[2, 3, 0, 1]] if r >= 8 else stored
     assert np.array_equal(back_k, kept.numpy()) and np.array_equal(back_e, words.numpy())
+
+
+@pytest.mark.parametrize("kind,epi,M,N,K,group,tile", [
+    (0, 3, 7000, 1280, 5120, 256, 17),   # grouped: 128x128 88 us, 64x64 111
+    (2, 3, 7000, 1280, 5120, 256, 17),   # 83, 110
+    (2, 3, 4500, 1280, 5120, 256, 17),   # 56.0, 57.8
+    (3, 1, 200, 5120, 1280, 1280, 7),    # bf16, two 64x64 tiles a CU: 11.2, 64x128 11.8
+    (3, 4, 512, 2560, 1280, 1280, 7),    # 10.9, 11.4
+    (3, 3, 1000, 1280, 1280, 1280, 7),   # 11.3, 11.8
+    (0, 0, 1500, 1280, 5120, 5120, 3),   # 64x128 19.2, 64x64 19.9
+    (2, 0, 1500, 1280, 5120, 5120, 3),   # 17.9, 18.6
+    (0, 0, 8401, 1280, 5120, 5120, 15),  # 256x256 on 16 waves 62.8, on 8 64.9
+    (0, 4, 8401, 2560, 1280, 1280, 9),   # 128x256 40.7, 256x256 45.4
+    (2, 3, 376, 1280, 5120, 256, 7), (2, 5, 3000, 5120, 1280, 1280, 10), (4, 8, 3000, 16384, 1024, 1024, 15)])
+def test_gemm_tile_choice(kind, epi, M, N, K, group, tile):
+    """The tile the cost model picks where another one was measured slower (microseconds beside the sizes)."""
+    from kernels.cuda_ext import ext
+
+    assert ext.gemm_tile(kind, epi, M, N, K, group) == tile
+
+
+def test_gemm_tile_choice_is_always_one_that_runs():
+    """Over odd sizes every product has a tile whose channels divide its own, one with grouped scales where they are,
+    and a forced tile without a kernel for the product is passed over."""
+    from kernels.cuda_ext import ext
+
+    widths = {0: 128, 3: 128, 4: 256, 5: 128, 6: 256, 7: 64, 8: 128, 9: 256, 10: 256, 15: 256, 17: 128}
+    try:
+        for forced in (-1, 0, 8, 14):
+            ext.set_gemm_tile(forced)
+            for M in (1, 63, 97, 1000, 9999):
+                for N in (64, 192, 256, 1280, 5120):
+                    for kind in range(4):
+                        tile = ext.gemm_tile(kind, 0, M, N, 1280, 1280)
+                        assert tile == forced or N % widths[tile] == 0, (forced, kind, M, N, tile)
+                        if kind < 3:
+                            assert ext.gemm_tile(kind, 3, M, N, 1280, 256) in (0, 3, 4, 5, 7, 8, 17)
+                assert ext.gemm_tile(4, 8, M, 256, 1024, 1024) in (3, 6, 9, 15, 17)
+    finally:
+        ext.set_gemm_tile(-1)
