@@ -111,6 +111,51 @@ def test_logmel_features(gpu, lengths):
     assert np.array_equal(bf16_bits(feats2), got)
 
 
+def test_logmel_batch_equals_pieces_alone(gpu):
+    """Each piece of a large batch has the bits that it has alone: over 33000 valid frames a wave takes eight frames in
+    turn (alone, one), crosses from piece to piece and over pieces without a frame; the normalisation holds up to 512
+    frames one way, more another, reads frames past 3072 again, and only the waves with frames take part (sizes at 32
+    and 512 frames and one either side, 3500 frames)."""
+    from kernels.features import Features
+
+    frames = [3001, 0, 1, 0, 0, 32, 33, 31, 511, 512, 513, 3072, 3073, 3500, 2, 160, 64, 65, *[2990] * 5, 1025]
+    frames += [3000] * 2 + [7] * 20 + [1500] * 2
+    lengths = [160 * n + (37 * i) % 160 for i, n in enumerate(frames)]
+    assert sum(frames) > 33000
+    fe = Features(device=gpu)
+    xs = [torch.from_numpy(x).to(gpu) for x in synthetic_audio(lengths, seed=5)]
+    feats, counts = fe(xs)
+    assert counts == [n + 1 for n in frames]
+    for i, x in enumerate(xs):
+        alone, _ = fe([x])
+        n = frames[i] + 1
+        assert torch.equal(feats[i, :n].view(torch.int16), alone[0].view(torch.int16)), frames[i]
+        assert (feats[i, n:] == 0).all(), frames[i]
+
+
+@pytest.mark.parametrize("frames", [513, 3200])
+def test_logmel_wide_bands_and_long_pieces(gpu, frames):
+    """Against the checker as above: a filter bank with a band of 41 bins, one of 16, one of 17 and an empty one, and
+    pieces of more frames than the normalisation holds."""
+    import types
+
+    from kernels.features import Features, default_extractor
+
+    mel = default_extractor().mel_filters.clone()
+    for band, (a, b) in {3: (20, 61), 70: (100, 116), 71: (100, 117), 90: (0, 0)}.items():
+        mel[band] = 0
+        mel[band, a:b] = torch.linspace(0.001, 0.02, b - a) if b > a else 0
+    fe = Features(types.SimpleNamespace(**{**vars(default_extractor()), "mel_filters": mel}), device=gpu)
+    xs = synthetic_audio([160 * frames + 11], seed=frames)
+    got = bf16_bits(fe(xs)[0])
+    want = oracle.logmel(np.concatenate(xs), [len(xs[0])], fe.window512.cpu().numpy(), fe.mel.cpu().numpy(),
+                         fe.band.cpu().numpy(), fe.preemphasis)
+    gf, wf = bf16_float(got), bf16_float(want)
+    tol = np.maximum(np.maximum(bf16_ulp(wf), bf16_ulp(gf)) * 1.0001, 1e-4)
+    assert (np.abs(gf - wf) <= tol).all()
+    assert (gf != wf).mean() <= 0.01
+
+
 def _stem_inputs(frames, seed):
     g = torch.Generator().manual_seed(seed)
     feats = torch.zeros(len(frames), max(frames), 128)
