@@ -744,10 +744,13 @@ extern "C" int cohere_logmel_features(const float* x, const int64_t* meta, int64
   // three frames)
   const int64_t per_wave = std::min<int64_t>(8, std::max<int64_t>(1, total_frames / (FPW * 1024)));
   const int64_t blocks = (total_frames + FPW * per_wave - 1) / (FPW * per_wave);
-  COHERE_REQUIRE(blocks < (1LL << 31) && pieces * (MELS / NB) < (1LL << 31), "logmel_features: too many frames");
+  COHERE_REQUIRE(blocks < (1LL << 31), "logmel_features: too many frames");
   logmel_kernel<<<(unsigned)blocks, FPW * 64, 0, s>>>(x, meta, (int)pieces, total_frames, (int)per_wave, window, mel,
                                                        band, preemph, work);
-  normalize_kernel<<<(unsigned)(pieces * (MELS / NB)), NTHR, 0, s>>>(work, meta + 2 * pieces, T, out);
+  constexpr int64_t most = (1LL << 17);  // a launch's threads are counted in 32 bits
+  for (int64_t p = 0; p < pieces; p += most)
+    normalize_kernel<<<(unsigned)(std::min(most, pieces - p) * (MELS / NB)), NTHR, 0, s>>>(
+        work, meta + 2 * pieces + p, T, out + p * T * MELS);
   return cohere::check_launch("logmel_features");
 }
 

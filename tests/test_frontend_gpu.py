@@ -251,3 +251,19 @@ def test_subsampling_with_pointwise(gpu, frames):
         b = gemm(b.view(-1, 256), *stem.pointwise[1], EPI_CONV_RELU).view(-1, 16, 256)
         _ext().sub_dw_pw(x, starts, dev(quarter), rows2, *stem.second_dw, *stem.pointwise[1], fbd)
         assert torch.equal(b.view(torch.int16), fbd.view(torch.int16)), shuffled
+
+
+def test_logmel_more_pieces_than_one_launch_holds(gpu):
+    """2^18 + 5 pieces of two frames each, on the same samples: every piece's features are the first one's (a launch
+    takes at most 2^32 threads, 2^14 of the normalisation's to a piece)."""
+    pieces, n, T = (1 << 18) + 5, 401, 3
+    x = torch.randn(n, generator=torch.Generator().manual_seed(2)).to(gpu)
+    from kernels.features import Features
+
+    fe = Features(device=gpu)
+    want, _ = fe([x])
+    meta = torch.cat([torch.zeros(pieces, dtype=torch.int64), torch.full((pieces,), n, dtype=torch.int64),
+                      2 * torch.arange(pieces + 1)]).to(gpu)
+    out = torch.zeros(pieces, T, 128, dtype=torch.bfloat16, device=gpu)
+    _ext().logmel_features(x, meta, 2 * pieces, fe.window512, fe.mel, fe.band, fe.preemphasis, out)
+    assert torch.equal(out, want.expand(pieces, T, 128))
