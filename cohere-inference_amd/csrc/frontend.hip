@@ -724,6 +724,22 @@ __global__ void __launch_bounds__(256) sub_dw_pw_kernel(const uint16_t* __restri
   pointwise<DWP_T * DWP_F, 4>(tile, wp, bp, out + (int64_t)i0 * DWP_F * PW_C, (int64_t)nt * DWP_F);
 }
 
+// ---- packed pieces ---------------------------------------------------------------------------------------------------
+// For packed pieces of count[b] rows each, every row's piece (its id) and its row within the piece. The counts travel as
+// kernel arguments: no upload, so nothing to pin, to wait for or to keep until a copy has run. A workgroup per piece.
+constexpr int PIECES = 128;  // of one launch
+struct Pieces {
+  int32_t id[PIECES], start[PIECES + 1];
+};
+__global__ void __launch_bounds__(256) piece_rows_kernel(const Pieces p, int32_t* __restrict__ piece_of,
+                                                         int32_t* __restrict__ row_of, int64_t stride) {
+  const int b = blockIdx.x, id = p.id[b], start = p.start[b], n = p.start[b + 1] - start;
+  for (int r = threadIdx.x; r < n; r += 256) {
+    piece_of[(start + r) * stride] = id;
+    row_of[(start + r) * stride] = r;
+  }
+}
+
 bool aligned(const void* q, int a) { return (reinterpret_cast<uintptr_t>(q) % a) == 0; }
 
 }  // namespace
@@ -812,4 +828,32 @@ extern "C" int cohere_sub_dw_pw(const uint16_t* x, const int32_t* in_start, cons
   sub_dw_pw_kernel<<<(unsigned)((n_rows + DWP_T - 1) / DWP_T), 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(
       x, in_start, in_len, rows, w, b, wp, bp, out, (int)n_rows);
   return cohere::check_launch("sub_dw_pw");
+}
+
+extern "C" int cohere_piece_rows(const int32_t* ids, const int32_t* counts, int64_t n, int32_t* piece_of, int32_t* row_of,
+                                 int64_t stride, void* stream) {
+  cohere::clear_error();
+  COHERE_REQUIRE(n >= 0 && stride >= 1, "piece_rows: bad sizes");
+  COHERE_REQUIRE(n == 0 || (counts && piece_of && row_of), "piece_rows: null pointer");
+  int64_t total = 0;
+  for (int64_t b = 0; b < n; ++b) {
+    COHERE_REQUIRE(counts[b] >= 0, "piece_rows: repeats can not be negative");
+    total += counts[b];
+  }
+  COHERE_REQUIRE(total < (1LL << 31), "piece_rows: too many rows");
+  int64_t row = 0;
+  for (int64_t b0 = 0; b0 < n; b0 += PIECES) {
+    const int m = (int)std::min<int64_t>(PIECES, n - b0);
+    Pieces p;
+    p.start[0] = 0;
+    for (int b = 0; b < m; ++b) {
+      p.id[b] = ids ? ids[b0 + b] : (int32_t)(b0 + b);
+      p.start[b + 1] = p.start[b] + counts[b0 + b];
+    }
+    if (p.start[m] > 0)
+      piece_rows_kernel<<<(unsigned)m, 256, 0, reinterpret_cast<hipStream_t>(stream)>>>(p, piece_of + row * stride,
+                                                                                        row_of + row * stride, stride);
+    row += p.start[m];
+  }
+  return cohere::check_launch("piece_rows");
 }

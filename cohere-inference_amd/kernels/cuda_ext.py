@@ -39,7 +39,8 @@ EXPORTS = ("cohere_gemm_i8", "cohere_gemm_sp", "cohere_quantize_rows", "cohere_l
            "cohere_logmel_features", "cohere_sub_conv0_dw", "cohere_sub_dw", "cohere_encoder_branch_workspace_bytes",
            "cohere_encoder_layers_noalloc", "cohere_dec_linear_fused", "cohere_dec_pick_embed",
            "cohere_gemm_sp_tiled", "cohere_pack_24_tiled_bytes", "cohere_pack_24_tiled", "cohere_sub_conv0_dw_pw",
-           "cohere_sub_dw_pw", "cohere_gemm_kv", "cohere_gemm_kv_q8", "cohere_gemm_tile")
+           "cohere_sub_dw_pw", "cohere_gemm_kv", "cohere_gemm_kv_q8", "cohere_gemm_tile",
+           "cohere_piece_rows")
 
 
 def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
@@ -81,6 +82,7 @@ def load_library(path: str = LIB_PATH) -> ctypes.CDLL:
         "cohere_sub_dw": [P, P, P, P, I64, P, P, P, I64, I64, P],
         "cohere_sub_conv0_dw_pw": [P, I64, P, P, I64, P, P, P, P, P, P, P, P],
         "cohere_sub_dw_pw": [P, P, P, P, I64, P, P, P, P, P, P],
+        "cohere_piece_rows": [P, P, I64, P, P, I64, P],
         "cohere_gemm_kv": [P, I64, P, P, I64, I64, P, P, P, P, I64, I64, I64, I64, P],
         "cohere_gemm_kv_q8": [P, I64, P, P, I64, I64, P, P, P, P, P, P, I64, I64, I64, I64, P],
         "cohere_encoder_layers": [P, I64, P, I64, P, P, I64, P, P, I64, I64, I64, ctypes.c_double, I32, I32, I32, P,
@@ -250,6 +252,23 @@ class _Ext:
             return
         self._call("cohere_sub_dw_pw", _ptr(x), _ptr(in_start), _ptr(in_len), _ptr(rows), n, _ptr(w), _ptr(b),
                    _ptr(wp), _ptr(bp), _ptr(out), _stream())
+
+    def piece_rows(self, ids, counts, piece_of, row_of):
+        """Of packed pieces of counts[b] rows: each row's ids[b] (None: b) into piece_of and its row within the piece into
+        row_of, int32 vectors on the GPU of sum(counts) values and one stride. The lists travel as kernel arguments."""
+        counts = [int(c) for c in counts]
+        ids = None if ids is None else [int(i) for i in ids]
+        _check(ids is None or len(ids) == len(counts), "piece_rows: one id per count")
+        _check(all(-2**31 <= v < 2**31 for v in counts + (ids or [])), "piece_rows: values beyond int32")
+        _check(all(c >= 0 for c in counts), "piece_rows: repeats can not be negative")
+        _check(piece_of.dtype == row_of.dtype == torch.int32 and piece_of.dim() == row_of.dim() == 1 and
+               piece_of.numel() == row_of.numel() == sum(counts), "piece_rows: int32 vectors of sum(counts) rows")
+        if not counts or piece_of.numel() == 0:
+            return
+        _check(piece_of.numel() == 1 or piece_of.stride(0) == row_of.stride(0) >= 1, "piece_rows: one stride")
+        host = ctypes.c_int32 * len(counts)
+        self._call("cohere_piece_rows", host(*ids) if ids is not None else None, host(*counts), len(counts),
+                   _ptr(piece_of), _ptr(row_of), max(1, piece_of.stride(0)), _stream())
 
     # ---- int8 GEMMs (bindings.cpp:41-43, 59-61) ----------------------------------------------------------------------
 

@@ -311,10 +311,9 @@ class SubsamplingStem:
     @staticmethod
     def _row_index(counts: list[int], dev) -> torch.Tensor:
         """int32 (sum(counts), 2): (piece, row within the piece) for every output row of a stage."""
-        c = torch.tensor(counts, dtype=torch.int64)
-        piece = torch.repeat_interleave(torch.arange(len(c)), c)
-        within = torch.arange(int(c.sum())) - torch.repeat_interleave(c.cumsum(0) - c, c)
-        return torch.stack([piece, within], 1).to(torch.int32).to(dev, non_blocking=True)
+        out = torch.empty(sum(counts), 2, device=dev, dtype=torch.int32)
+        ext.piece_rows(None, counts, out[:, 0], out[:, 1])
+        return out
 
     @torch.no_grad()
     def __call__(self, features: torch.Tensor, frames: list[int]) -> tuple[torch.Tensor, list[int]]:

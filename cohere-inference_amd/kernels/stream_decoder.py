@@ -388,10 +388,8 @@ class StreamDecoder:
             out = torch.empty(rows, self.proj[0].shape[0], device=hidden.device, dtype=hidden.dtype)
             ext.gemm(mem, self.proj[0], self.proj[1], out, EPI_BIAS, None, 1.0, 8)
             mem = out
-        where = torch.empty(2, rows, dtype=torch.int32)
-        where[0] = torch.repeat_interleave(torch.tensor(slots, dtype=torch.int32), torch.tensor(lengths))
-        where[1] = torch.cat([torch.arange(n, dtype=torch.int32) for n in lengths])
-        where = where.pin_memory().to(hidden.device, non_blocking=True)
+        where = torch.empty(2, rows, device=hidden.device, dtype=torch.int32)
+        ext.piece_rows(slots, lengths, where[0], where[1])
         ext.gemm_kv(mem, self.cross_w, self.cross_b, where[0], where[1], self.cross_k, self.cross_v, self.cross_ks,
                     self.cross_vs)
 

@@ -350,6 +350,13 @@ int cohere_sub_dw_pw(const uint16_t* x, const int32_t* in_start, const int32_t* 
                      int64_t n_rows, const float* w, const float* b, const uint16_t* wp, const uint16_t* bp,
                      uint16_t* out, void* stream);
 
+/* Index tables of packed pieces (the reference builds them with torch on the host and uploads them,
+ * kernels/stream_decoder.py:216-238, kernels/fast_encoder.py:185-202): ids (null: 0 .. n - 1) and counts are HOST arrays
+ * of n pieces, read before the call returns; row i of the packed rows gets its piece's id in piece_of[i * stride] and its
+ * row within the piece in row_of[i * stride] (device memory). */
+int cohere_piece_rows(const int32_t* ids, const int32_t* counts, int64_t n, int32_t* piece_of, int32_t* row_of,
+                      int64_t stride, void* stream);
+
 /* The last error on this thread ("" when none). */
 const char* cohere_last_error(void);
 

@@ -447,3 +447,49 @@ def test_gemm_kv_at_every_tile(gpu, rows, L, H, K, q8):
                 assert torch.equal(x, y), tile
     finally:
         _ext().set_gemm_tile(-1)
+
+
+@pytest.mark.parametrize("pieces", [1, 127, 128, 129, 300])
+def test_piece_rows(gpu, pieces):
+    """Index tables of packed pieces against torch's, pieces without rows among them, one to three launches; as two
+    vectors and as the columns of one table, nothing written past either."""
+    g = torch.Generator().manual_seed(pieces)
+    counts = (torch.randint(0, 600, (pieces,), generator=g) * (torch.rand(pieces, generator=g) < 0.8)).tolist()
+    counts[-1] += 1
+    ids = torch.randint(-5, 1 << 20, (pieces,), generator=g).tolist()
+    n = sum(counts)
+    row = torch.cat([torch.arange(c) for c in counts]).int()
+    for names in (ids, None):
+        piece = torch.repeat_interleave(torch.tensor(ids if names else range(pieces)), torch.tensor(counts)).int()
+        two = torch.full((2, n + 1), -9, dtype=torch.int32, device=gpu)
+        _ext().piece_rows(names, counts, two[0, :n], two[1, :n])
+        assert torch.equal(two[:, :n].cpu(), torch.stack([piece, row])) and (two[:, n] == -9).all()
+        table = torch.full((n + 1, 3), -9, dtype=torch.int32, device=gpu)
+        _ext().piece_rows(names, counts, table[:n, 0], table[:n, 1])
+        assert torch.equal(table[:n, :2].cpu(), torch.stack([piece, row], 1))
+        assert (table[n] == -9).all() and (table[:, 2] == -9).all()
+
+
+def test_fill_cross_uploads_nothing(gpu, monkeypatch):
+    """A fill takes no pinned memory and no copy from the host: with either the GPU waits between the two products of a
+    fill on its own (a new pinned block is an allocation, milliseconds). Refusals as before."""
+    from kernels.stream_decoder import StreamDecoder
+
+    model = make_decoder(hidden=512, heads=4, layers=1, ffn=512, vocab=512, seed=15, device=gpu, dtype=torch.bfloat16)
+    dec = StreamDecoder(model, slots=4, max_new_tokens=8, max_prompt=4, buckets=(4,), int8=False, frames=8,
+                        capture=False)
+    mem = torch.randn(16, 512, generator=torch.Generator().manual_seed(16)).to(torch.bfloat16).to(gpu)
+
+    def refuse(*a, **k):
+        raise AssertionError("a host copy in fill_cross")
+
+    with monkeypatch.context() as m:
+        for name in ("pin_memory", "to", "cuda", "copy_"):
+            m.setattr(torch.Tensor, name, refuse)
+        dec.fill_cross(mem, [8, 3, 5], [2, 0, 1])
+    kv = (mem.float() @ dec.cross_w.float().T + dec.cross_b.float())
+    want = kv[8:11, :128]  # the second piece's keys of head 0, slot 0
+    assert torch.allclose(dec.cross_k[0, 0, 0, :3].float(), want, atol=0.05, rtol=0.02)
+    for lengths, slots in (([8, 3], [2, 0]), ([8, 8], [1]), ([17, -1], [0, 1])):
+        with pytest.raises(RuntimeError):
+            dec.fill_cross(mem, lengths, slots)

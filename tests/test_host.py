@@ -216,3 +216,19 @@ def test_gemm_tile_choice_is_always_one_that_runs():
                 assert ext.gemm_tile(4, 8, M, 256, 1024, 1024) in (3, 6, 9, 15, 17)
     finally:
         ext.set_gemm_tile(-1)
+
+
+def test_piece_rows_rejects():
+    """Refused before any launch, as torch.repeat_interleave refused them."""
+    from kernels.cuda_ext import _lib as lib
+    from kernels.cuda_ext import ext
+
+    t = torch.empty(5, dtype=torch.int32)
+    for ids, counts, match in (([1], [2, 3], "one id"), ([1, 2], [6, -1], "negative"), ([1, 2], [2, 2], "sum"),
+                               ([1 << 31, 0], [2, 3], "int32"), (None, [5, 1], "sum")):
+        with pytest.raises(RuntimeError, match=match):
+            ext.piece_rows(ids, counts, t, t)
+    ext.piece_rows([], [], t[:0], t[:0])
+    counts = (ctypes.c_int32 * 2)(3, -3)
+    rc, msg = _raw(lib, "cohere_piece_rows", None, counts, 2, 1 << 20, 1 << 20, 1, None)
+    assert rc != 0 and "negative" in msg
