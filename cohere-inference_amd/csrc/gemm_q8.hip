@@ -29,9 +29,10 @@ int num_cus() {
 // 1.3 times as long, and what is more than that counts by half rounds. (As whole rounds of two with one workgroup's
 // time, 7000 grouped rows x 1280 x 5120 took 64x64 tiles, 110 us, where 128x128 ones take 83.)
 // Fitted to graph replays of the encoder's linears at 376, 1892, 3000 and 8416 rows (K 1280 and 5120) and the bf16 stem,
-// cross-attention and layer shapes. Every tile timed for 18 linears (int8, 2:4, grouped, bf16) at 32 row counts from 6 to
-// 9024: the choice is within 4 % of the fastest tile at 549 of 561 points (the rest are bf16, the worst 1280 x 1280 over
-// 7000 rows and more, 14 %), and nowhere slower than the former rule's beyond the noise of 2 %. Against that, the largest
+// cross-attention and layer shapes. Every tile timed for 18 linears (int8, 2:4, grouped, bf16) at 48 row counts from 6 to
+// 9024: the choice is within 4 % of the fastest tile at all but 19 of 849 points (18 of them bf16, the worst 1280 x 1280
+// over 7000 rows and more, 14 %) and EIGHT_WAVES' products, and nowhere slower than the former rule's beyond the noise.
+// Against that, the largest
 // tile that gives 64 % of the CUs a workgroup (the former rule): bf16 1892 x 1280 x 5120 62.2 -> 39.1 us, 1892 x 5120 x
 // 1280 SILU 48.3 -> 39.7, 1892 x 1280 x 1280 21.4 -> 13.9, 3000 x 1024 x 1280 15.0 -> 12.6; int8 3000 x 1280 x 1280 12.2
 // -> 9.5, grouped 1892 x 1280 x 5120 42.7 -> 28.3.
@@ -46,6 +47,12 @@ constexpr TileCost BF16_COST[] = {{6, 1, 1.28, 10.9, 0.0}, {15, 1, 1.335, 10.0, 
 constexpr TileCost DENSE_COST[] = {{6, 1, 1.28, 10.9, 8.0}, {15, 1, 1.285, 10.5, 6.2}, {8, 1, .695, 7.5, 3.0},
                                    {9, 1, .69, 6.6, 3.0},   {17, 1, .42, 4.5, 2.0},    {4, 1, .6, 4.0, 3.3},
                                    {3, 1, .335, 3.3, 2.0},  {5, 1, .27, 3.1, 2.0},     {7, 2, .265, 3.0, 2.0}};
+// int8 over several rounds: alone the 8-wave tiles (doubled fragments) are up to 10 % faster than 256x256 on 16 waves, but
+// whole layers that ran on them were up to 4 % slower, kernels that had not changed among them (2 blocks of 16 clips of
+// 200 to 376 frames 835 -> 860 us, of 24 x 376 1356 -> 1378; the attention 40.7 -> 44.9, the depthwise convolution 18.6 ->
+// 19.2): the chip's clock falls under the denser matrix work. Counted a quarter longer such products keep the 256x256
+// tile: 836 and 1355 us. (Over one round they stay: 8 x 375 frames 522 -> 509. bf16 layers gained at every size.)
+constexpr double EIGHT_WAVES = 1.25;
 // 2:4 weights; 10 reads stage-tiled records (row-major ones take 15)
 constexpr TileCost SPARSE_COST[] = {{10, 1, 1.03, 11.2, 7.0}, {15, 1, 1.25, 11.0, 7.0}, {8, 1, .58, 6.2, 3.5},
                                     {9, 1, .52, 6.7, 3.5},    {17, 1, .47, 2.6, 2.0},   {0, 1, .437, 3.6, 2.0},
@@ -71,13 +78,15 @@ int choose_tile(const GemmArgs& p, bool grouped, bool bf = false) {
   const int64_t cus = num_cus();
   int best = -1;
   double least = 0.0;
+  const bool dense = !grouped && !p.E && !bf;
   auto consider = [&](const auto& table) {
     for (const TileCost& t : table) {
       if (!fits(t.id) || (p.E && !p.tiled && t.id == 10)) continue;
       const int64_t n = (int64_t)((p.M + TILES[t.id].bm - 1) / TILES[t.id].bm) * (p.N / TILES[t.id].bn);
       const double rounds = (double)((n + cus - 1) / cus), once = t.f + (p.epi == EPI_SILU_Q8 ? t.q8 : 0.0);
-      const double us = t.per_cu == 1 || n <= cus ? rounds * (t.c * stages + once)
-                                                  : rounds / 2 * (1.3 * t.c * stages + once);
+      double us = t.per_cu == 1 || n <= cus ? rounds * (t.c * stages + once)
+                                            : rounds / 2 * (1.3 * t.c * stages + once);
+      if (dense && n > cus && (t.id == 8 || t.id == 9 || t.id == 17)) us *= EIGHT_WAVES;
       if (best < 0 || us < least) best = t.id, least = us;
     }
   };

@@ -188,7 +188,9 @@ def test_pack_24_tiled_matches_c_abi_and_round_trips():
     (0, 0, 1500, 1280, 5120, 5120, 3),   # 64x128 19.2, 64x64 19.9
     (2, 0, 1500, 1280, 5120, 5120, 3),   # 17.9, 18.6
     (0, 0, 8401, 1280, 5120, 5120, 15),  # 256x256 on 16 waves 62.8, on 8 64.9
-    (0, 4, 8401, 2560, 1280, 1280, 9),   # 128x256 40.7, 256x256 45.4
+    (0, 4, 8401, 2560, 1280, 1280, 15),  # several rounds, int8: whole layers are faster on 256x256
+    (0, 0, 4601, 3840, 1280, 1280, 15), (0, 5, 4601, 5120, 1280, 1280, 15),  # 2 blocks 836 us, on 128x256 860
+    (0, 4, 3000, 2560, 1280, 1280, 9),   # one round: 13.4, 17.4
     (2, 3, 376, 1280, 5120, 256, 7), (2, 5, 3000, 5120, 1280, 1280, 10), (4, 8, 3000, 16384, 1024, 1024, 15)])
 def test_gemm_tile_choice(kind, epi, M, N, K, group, tile):
     """The tile the cost model picks where another one was measured slower (microseconds beside the sizes)."""
