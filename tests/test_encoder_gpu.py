@@ -250,3 +250,20 @@ def test_encoder_layers_few_rows(gpu, lengths, sparse, sparse_w1):
     few = layers(x[:sum(lengths)].clone(), lengths)
     many = layers(x.clone(), [*lengths, 100])[:sum(lengths)]
     assert np.array_equal(_bits(few), _bits(many))
+
+
+@pytest.mark.parametrize("lengths,heads,tiled", [([26, 17], 8, True), ([96], 16, False), ([33], 8, False), ([1], 8, False)])
+def test_encoder_layers_few_rows_forms(gpu, lengths, heads, tiled):
+    """The same for 8 heads and for row-major 2:4 weights (kept values and selectors in two tensors), which the few-row
+    launches read by paths of their own."""
+    layers = product_layers(gpu, 1, 43, True, True, heads=heads)
+    if not tiled:
+        for ly in layers.layers:
+            ly.tiled = {}
+        layers.layer_tensors = [ly.fields() for ly in layers.layers]
+    g = torch.Generator().manual_seed(sum(lengths) + heads)
+    x = torch.randn(sum(lengths) + 100, 1280, generator=g).to(torch.bfloat16).to(gpu)
+    print(f"few rows {lengths} heads {heads} tiled {tiled}", flush=True)
+    few = layers(x[:sum(lengths)].clone(), lengths)
+    many = layers(x.clone(), [*lengths, 100])[:sum(lengths)]
+    assert np.array_equal(_bits(few), _bits(many))

@@ -60,6 +60,38 @@ def test_gemm_bf16(gpu, M, N, K, epi):
         assert_bf16_close(bf16_bits(out), want, max_frac=0.02)
 
 
+@pytest.mark.parametrize("K", [1280, 1312])
+@pytest.mark.parametrize("epi", list(EPIS))
+def test_gemm_bf16_at_every_tile(gpu, epi, K):
+    """Every bf16 tile adds K in the same order: the same bits whichever is forced, with more K stages than a tile's ring
+    holds (1312: and a half one) and rows that fill no tile; one of them, 8 waves of doubled fragments, to the checker's
+    bar."""
+    M, N, e = 300, 512, EPIS[epi]
+    g = torch.Generator().manual_seed(K + e)
+    a = torch.randn(M, K, generator=g).to(torch.bfloat16)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16)
+    b = (torch.randn(N, generator=g) * 0.1).to(torch.bfloat16)
+    r = torch.randn(M, N, generator=g).to(torch.bfloat16)
+    ad, wd, bd, outs = a.to(gpu), w.to(gpu), b.to(gpu), {}
+    try:
+        for tile in range(-1, _ext().set_gemm_tile(-1)):
+            _ext().set_gemm_tile(tile)
+            print(f"bf16 {epi} K={K} tile {tile}", flush=True)
+            out = r.to(gpu) if e == 3 else torch.empty(M, N // 2 if e == 4 else N, dtype=torch.bfloat16, device=gpu)
+            _ext().gemm(ad, wd, bd, out, e, out if e == 3 else None, 0.5, 8)
+            outs[tile] = bf16_bits(out)
+    finally:
+        _ext().set_gemm_tile(-1)
+    for tile, bits in outs.items():
+        assert np.array_equal(bits, outs[9]), tile
+    want = oracle.gemm_bf16(bf16_bits(a), bf16_bits(w), bf16_bits(b), e, resid=bf16_bits(r), alpha=0.5)
+    got_f, want_f = bf16_float(outs[9]).astype(np.float64), bf16_float(want).astype(np.float64)
+    # test_gemm_bf16's bars: one ulp, or two roundings in a row (SILU, GLU, CONV_RELU) two
+    ulps = 2.0001 if e in (1, 4, 6) else 1.0001
+    assert (np.abs(got_f - want_f) <= np.maximum(1e-2 * np.sqrt(np.mean(want_f ** 2)), ulps * bf16_ulp(want_f))).all()
+    assert (outs[9] != want).mean() <= 0.02
+
+
 def test_gemm_bf16_strided_rows_and_no_bias(gpu):
     g = torch.Generator().manual_seed(3)
     big = torch.randn(200, 640, generator=g).to(torch.bfloat16)
