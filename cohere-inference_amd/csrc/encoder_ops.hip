@@ -254,11 +254,12 @@ relpos_attention_kernel(const AttnArgs p) {
   // (64 chunks each) of keys, as many of table rows, and VSL pairs of wave loads of values, dealt to the four waves in
   // that order, SL each: every wave issues the same loads with no branch between them, so no wait for an earlier load
   // is needed among them (with loads under per-thread conditions the compiler put one there, a memory latency in each
-  // tile of every wave that fetched values). With the ring's first rows loaded in one go as well, head size 160 over
-  // one 376-frame clip of 8 heads went from 30.3 to 24.6 us and over 8 clips from 30.7 to 25.1; head size 80, with three
-  // workgroups a CU to cover such waits, from 31.7 to 31.1 over 8 clips of 375 frames. A load's chunk is (row id / CH, chunk id % CH) for keys and table rows;
-  // for values it is (key pair item % 16, chunk item / 16), so that the pair's 8 dims go to LDS as 8 dwords of the
-  // transposed tile with the lanes of a wave on distinct banks. 32-bit element offsets from uniform bases (a layer's
+  // tile of every wave that fetched values). With the ring's first rows loaded in one go as well, in graphs of its own:
+  // head size 160 (8 heads) over one 376-frame clip 26.3 -> 24.1 us, 8 clips 38.1 -> 35.3, 24 clips 94.0 -> 79.7, one clip
+  // of 26 frames 6.0 -> 6.2; head size 80, with three workgroups a CU to cover such waits, 30.9 -> 30.6 over 8 clips of
+  // 375. A load's chunk is (row id / CH, chunk id % CH) for keys and table rows; for values it is (key pair item % 16,
+  // chunk item / 16), so that the pair's 8 dims go to LDS as 8 dwords of the transposed tile with the lanes of a wave on
+  // distinct banks. 32-bit element offsets from uniform bases (a layer's
   // qkv and table stay below 2^31 elements); keys past the sequence load its last key (their scores are masked and
   // their probabilities exactly 0, the values finite, so no register is zeroed) and table rows are clamped to the
   // table.

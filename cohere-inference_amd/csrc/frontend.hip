@@ -44,8 +44,10 @@ DEVI int piece_of(const int64_t* frame_start, int pieces, int64_t f) {
   return lo;
 }
 
-// Bound by vector-instruction issue: about 1000 instructions a frame, 4 cycles each (12,800 frames: 21 us of issue over
-// the 1024 SIMDs, 28 us measured, 29 with one frame per wave, tables per frame and a branch around each sample load).
+// Bound by no one unit: over 12,800 frames (27.8 us; 29 with one frame per wave, tables per frame and a branch around each
+// sample load) the counters give 600 vector instructions a frame, a wave's tables among them, 4 cycles each: 12.5 us of
+// issue over the 1024 SIMDs, 45 %; the 15 MB take 3 us. The rest is latency: a wave's passes one after another through
+// LDS, and its first samples and tables.
 // A wave takes `per_wave` consecutive frames, so that the twiddle table (computed in double) and the mel weights in LDS
 // are made once for FPW * per_wave frames; the samples of its next frame are loaded while one is transformed. Its
 // FFT buffers are its own: between the passes it waits for its own LDS accesses only.

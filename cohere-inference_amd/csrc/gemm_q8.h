@@ -99,7 +99,6 @@ struct Tile {
   static constexpr int KSTEP = MS == 16 ? (SPARSE ? 128 : 64) : (SPARSE ? 64 : 32);
   static constexpr int SPS = 128 / KSTEP;
   static constexpr int RPL = MS == 16 ? 4 : 16;
-  // fragment double-buffering (register budget): up to 4 waves, or 8 waves of small tiles
   // fragment double-buffering where the registers allow it: up to 4 waves, or 8 waves of small tiles (bf16 128x256
   // tiles 64.1 -> 47 us at 3008 x 1280 x 4096, int8 GLU at 3000 x 2560 x 1280 17.4 -> 13.4); not with grouped scales
   // (8 waves of 128x128, 2:4: 29.2 -> 31.8 us)
@@ -828,6 +827,8 @@ void launch_tile(const GemmArgs& args, hipStream_t s) {
 //   13 128x256 (2x2, 3)   14 256x256 (2x2, 2 dense / 3 sparse)   15 256x256 (4x4: 16 waves, 2 dense / 3 sparse)
 //   16 128x128 (4x2: 8 waves of 32 tokens x 64 channels, 4)   17 128x128 (2x4: 8 waves of 64 tokens x 32 channels, 4);
 //   tiles 11-13 use the 32x32 matrix instructions, the others 16x16
+// The choice by shape takes 3, 4, 5, 7, 8, 9, 15, 17, dense 6, sparse 0 and 10 (gemm_q8.hip's cost tables); the others are
+// there for cohere_set_gemm_tile only.
 struct TileInfo {
   int bm, bn;
   bool grouped_ok;

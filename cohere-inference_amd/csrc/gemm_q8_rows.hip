@@ -238,7 +238,7 @@ void launch_ns(const Args& p, hipStream_t s) {
   int nw = units < MAX_WAVES ? units : MAX_WAVES;
   while (units % nw) --nw;
   if (nw < 4 && units >= 4) nw = 4;
-    constexpr int UB = BF ? 1 : 2;
+  constexpr int UB = BF ? 1 : 2;
   const size_t lds = ((GROUPED ? units : nw) * 16 * (NS * 16 + 4) + 16 * (GROUPED ? units : 1) + nw * 16) * 4;
   rows_gemm_kernel<XM, SPARSE, EPI, NS, UB>
       <<<dim3(p.N / (16 * NS), (p.M + 15) / 16), nw * 64, lds, s>>>(p);
