@@ -188,9 +188,9 @@ bool al16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
 
 // Whether the few-row launch sequence takes this call: few rows, 256-column feed-forward groups, and every argument
 // one that the general sequence would accept (it words the refusals).
-bool few_rows(const uint16_t* x, int64_t rows, const void* const* fields, int64_t n_layers, int64_t group,
-              int64_t c_i8, int64_t c_grp, int64_t c_ff1, int64_t c_pw1, int64_t c_o, int64_t c_sp) {
-  if (rows > cohere_rows_gemm::ROWS_MAX || group != cohere_rows_gemm::UNIT || !al16(x)) return false;
+bool few_rows(const uint16_t* x, int64_t rows, const void* workspace, const void* const* fields, int64_t n_layers,
+              int64_t group, int64_t c_i8, int64_t c_grp, int64_t c_ff1, int64_t c_pw1, int64_t c_o, int64_t c_sp) {
+  if (rows > cohere_rows_gemm::ROWS_MAX || group != cohere_rows_gemm::UNIT || !al16(x) || !al16(workspace)) return false;
   for (int64_t c : {c_i8, c_grp, c_pw1, c_o})
     if (cohere_gemm::ref_config_group((int)c) == -2) return false;
   if (c_sp < -1 || c_sp > 4 || cohere_gemm::ref_config_group((int)c_ff1) != group) return false;
@@ -345,7 +345,7 @@ extern "C" int cohere_encoder_layers(uint16_t* x, int64_t rows, const void* cons
                        ": a feed-forward linear has neither dense nor 2:4 weights");
   }
 
-  if (few_rows(x, rows, fields, n_layers, group, c_i8, c_grp, c_ff1, c_pw1, c_o, c_sp))
+  if (few_rows(x, rows, workspace, fields, n_layers, group, c_i8, c_grp, c_ff1, c_pw1, c_o, c_sp))
     return encoder_layers_few(x, rows, fields, n_layers, eps, tiles, n_tiles, lo, hi, rel_off, max_len, rel_rows, scale,
                               heads, head_dim, c_i8, c_pw1, c_o, ws, stream);
   const int64_t ts_ld = DFF / group;

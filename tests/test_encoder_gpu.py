@@ -267,3 +267,23 @@ def test_encoder_layers_few_rows_forms(gpu, lengths, heads, tiled):
     few = layers(x[:sum(lengths)].clone(), lengths)
     many = layers(x.clone(), [*lengths, 100])[:sum(lengths)]
     assert np.array_equal(_bits(few), _bits(many))
+
+
+@pytest.mark.parametrize("rows", [26, 96, 97])
+def test_encoder_layers_refuses_a_misaligned_workspace(gpu, rows):
+    """A workspace at 8 bytes past 16: refused at any number of rows (the few-row launches copy 16-byte chunks of it),
+    the rows as they were."""
+    from kernels.cuda_ext import ext
+    from kernels.fast_encoder import metadata
+
+    layers = product_layers(gpu, 1, 47, True)
+    x = torch.randn(rows, 1280, generator=torch.Generator().manual_seed(rows)).to(torch.bfloat16).to(gpu)
+    before, meta = x.clone(), metadata([rows], gpu)
+    args, cfg = ext._encoder_args(x, layers.layer_tensors, layers.layer_eps, meta["tiles"], meta["lo"], meta["hi"],
+                                  layers.rel_off, meta["max_len"], layers.scale, layers.int8, layers.configs(rows))
+    nbytes = int(ext._lib.cohere_encoder_branch_workspace_bytes(rows, cfg[4], 1))
+    ws = torch.empty(nbytes + 8, dtype=torch.uint8, device=gpu)
+    with pytest.raises(RuntimeError, match="aligned"):
+        ext._call("cohere_encoder_layers", *args, ws.data_ptr() + 8, nbytes, torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(x.view(torch.int16), before.view(torch.int16))
