@@ -251,7 +251,7 @@ def test_subsampling_with_pointwise(gpu, frames):
     """The convolutions with their pointwise convolution in one launch give the separate launches' bits: full and partial
     groups of four output rows, groups that span pieces (rows not consecutive), and rows in any order; weights of 24
     significant bits as bf16 ones, mel values over sixteen powers of two (where sums in another order round
-    differently), and an infinite and a NaN mel value."""
+    differently), an infinite and a NaN mel value, and subnormal mel values that nothing covers (no biases)."""
     from kernels.cuda_ext import EPI_CONV_RELU
     from kernels.fast_encoder import SubsamplingStem, gemm
 
@@ -269,11 +269,14 @@ def test_subsampling_with_pointwise(gpu, frames):
         bad = fb.clone()
         bad[0, frames[0] // 2, 40], bad[0, frames[0] // 3, 90] = float("inf"), float("nan")
         spread = (fb.float() * torch.exp2(torch.randint(-8, 9, fb.shape, generator=g).to(gpu))).to(torch.bfloat16)
-        for first, x in ((stem.first, fb), (wide, fb), (wide, spread), (stem.first, spread), (stem.first, bad)):
+        pw, none = stem.pointwise[0], torch.zeros(256, device=gpu)
+        bare, tiny = (stem.first[0], none, stem.first[2], none), (fb.float() * 2.0 ** -128).to(torch.bfloat16)
+        for first, pw, x in ((stem.first, pw, fb), (wide, pw, fb), (wide, pw, spread), (stem.first, pw, spread),
+                             (stem.first, pw, bad), (bare, (pw[0], none.to(torch.bfloat16)), tiny)):
             a, fa = (torch.empty(len(rows1), 32, 256, dtype=torch.bfloat16, device=gpu) for _ in range(2))
             _ext().sub_conv0_dw(x, dev(frames), rows1, *first, a)
-            a = gemm(a.view(-1, 256), *stem.pointwise[0], EPI_CONV_RELU).view(-1, 32, 256)
-            _ext().sub_conv0_dw_pw(x, dev(frames), rows1, *first, *stem.pointwise[0], fa)
+            a = gemm(a.view(-1, 256), *pw, EPI_CONV_RELU).view(-1, 32, 256)
+            _ext().sub_conv0_dw_pw(x, dev(frames), rows1, *first, *pw, fa)
             nan = torch.isnan(a)
             assert torch.equal(nan, torch.isnan(fa))
             assert torch.equal(a[~nan].view(torch.int16), fa[~nan].view(torch.int16)), shuffled
