@@ -677,7 +677,7 @@ __global__ void __launch_bounds__(WM* WN * 64) gemm_q8_kernel(const GemmArgs p) 
         if constexpr (KV) {
           // the chunk's 128-vector: 16 consecutive lanes of one row hold it (m is theirs together). Bound by the
           // product; writing the caches here saves the product's write and read (98 MB each at 3000 rows of 16384):
-          // the whole fill of 8 x 375 frames 177 -> 147 us
+          // the whole fill of 8 x 375 frames 177 -> 147 us (123 with the slots and positions written by a kernel)
           const int cb = (oc0 >> 7) + (cc >> 4), d8 = cc & 15, hd = cb % p.H, kvi = cb / p.H % 2, l = cb / p.H / 2;
           const int64_t vec = (((int64_t)l * p.S + p.slot_of[m]) * p.H + hd) * p.T + p.frame_of[m];
           if constexpr (EPI == EPI_KV) {

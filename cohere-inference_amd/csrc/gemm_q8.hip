@@ -51,7 +51,9 @@ constexpr TileCost DENSE_COST[] = {{6, 1, 1.28, 10.9, 8.0}, {15, 1, 1.285, 10.5,
 // whole layers that ran on them were up to 4 % slower, kernels that had not changed among them (2 blocks of 16 clips of
 // 200 to 376 frames 835 -> 860 us, of 24 x 376 1356 -> 1378; the attention 40.7 -> 44.9, the depthwise convolution 18.6 ->
 // 19.2): the chip's clock falls under the denser matrix work. Counted a quarter longer such products keep the 256x256
-// tile: 836 and 1355 us. (Over one round they stay: 8 x 375 frames 522 -> 509. bf16 layers gained at every size.)
+// tile: 836 and 1355 us. How much it is depends on the card: with the GLU product of 8401 rows on 128x256 a block took 628
+// us against 632 on one, and on another 666 where the former rule took 657. (Over one round they stay: 8 x 375 frames
+// 522 -> 509. bf16 layers gained at every size.)
 constexpr double EIGHT_WAVES = 1.25;
 // 2:4 weights; 10 reads stage-tiled records (row-major ones take 15)
 constexpr TileCost SPARSE_COST[] = {{10, 1, 1.03, 11.2, 7.0}, {15, 1, 1.25, 11.0, 7.0}, {8, 1, .58, 6.2, 3.5},
