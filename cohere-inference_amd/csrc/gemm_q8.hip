@@ -113,7 +113,7 @@ int ref_cfg_group(int cfg) {
 // Few rows go to the few-row kernel where it is the faster one (the same bits; a forced tile keeps the tile GEMM)
 bool rows_gemm(const GemmArgs& p, bool sparse, bool grouped, hipStream_t s) {
   namespace R = cohere_rows_gemm;
-  if (g_tile_override >= 0 || !R::better_than_tiles(p.M, p.N, p.K)) return false;
+  if (g_tile_override >= 0 || !R::better_than_tiles(p.M, p.N, p.K, grouped)) return false;
   if (p.epi != EPI_BIAS && p.epi != EPI_RESID && p.epi != EPI_GLU) return false;
   if (grouped && p.group != R::UNIT) return false;
   R::Args a{};

@@ -37,7 +37,7 @@ struct Args {
 // whether the kernel takes these sizes at all (alignments as the tile GEMM's)
 bool fits(int64_t M, int64_t N, int64_t K);
 // whether it is also the faster one for int8 rows
-bool better_than_tiles(int64_t M, int64_t N, int64_t K);
+bool better_than_tiles(int64_t M, int64_t N, int64_t K, bool grouped);
 // launches it; epi: the EPI_* ids BIAS, RESID, GLU (RESID only unless X_Q8). false when there is no such kernel
 bool launch(XMode xm, bool sparse, int epi, const Args& p, hipStream_t s);
 

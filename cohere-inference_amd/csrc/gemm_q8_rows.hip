@@ -234,10 +234,12 @@ template <int XM, bool SPARSE, int EPI, int NS>
 void launch_ns(const Args& p, hipStream_t s) {
   constexpr bool GROUPED = XM == X_Q8G || XM == X_BFG, BF = XM == X_BF || XM == X_BFG;
   const int units = p.K / UNIT;
-  // waves: one unit each up to MAX_WAVES, else as many as share the units evenly
+  // waves: one unit each up to MAX_WAVES, else as many as share the units evenly; at least 4, units or not, so that a
+  // thread has one output and the residual's old value is one memory round trip (with one wave four in a row: K 256,
+  // 32 x 1280 with residual 4.3 us, the tiles 3.3)
   int nw = units < MAX_WAVES ? units : MAX_WAVES;
   while (units % nw) --nw;
-  if (nw < 4 && units >= 4) nw = 4;
+  if (nw < 4 && !one_unit(XM)) nw = 4;
   constexpr int UB = BF ? 1 : 2;
   const size_t lds = ((GROUPED ? units : nw) * 16 * (NS * 16 + 4) + 16 * (GROUPED ? units : 1) + nw * 16) * 4;
   rows_gemm_kernel<XM, SPARSE, EPI, NS, UB>
@@ -261,9 +263,12 @@ bool fits(int64_t M, int64_t N, int64_t K) {
 
 // Up to ROWS_MAX rows. Against the 64 x 64 tile, whose time is its K stages (about 3 us + 0.33 us per 128 K) at any few
 // rows, this kernel's grows with its workgroups: N 1280, K 1280 5.1 us against 5.8 at 32 rows, 7.8 against 5.8 at 64;
-// N 3840, K 1280 7.0 against 5.4 at 26 rows; K 5120 (grouped) 9.5 against 16.2 at 26 and at 64 rows.
-bool better_than_tiles(int64_t M, int64_t N, int64_t K) {
-  return M <= ROWS_MAX && fits(M, N, K) && N / 16 * ((M + 15) / 16) <= (K < 2560 ? 192 : 512);
+// N 3840, K 1280 7.0 against 5.4 at 26 rows; K 5120 (grouped) 9.5 against 16.2 at 26 and at 64 rows. From K 3072 on it
+// is the faster one at every size up to 512 workgroups (N 256 .. 5120, 1 to 96 rows: 0.37 to 1.01 of the tiles' time);
+// K 2560 with scales per row beyond 256 workgroups, two strips each, 8.4 us against 7.4.
+bool better_than_tiles(int64_t M, int64_t N, int64_t K, bool grouped) {
+  const int64_t most = K < 2560 ? 192 : K < 3072 && !grouped ? 256 : 512;
+  return M <= ROWS_MAX && fits(M, N, K) && N / 16 * ((M + 15) / 16) <= most;
 }
 
 bool launch(XMode xm, bool sparse, int epi, const Args& p, hipStream_t s) {

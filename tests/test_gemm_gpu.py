@@ -372,10 +372,11 @@ def test_empty_rows_noop(ext):
 # ---- few rows: the kernel of csrc/gemm_q8_rows.hip ----------------------------------------------------------------------
 
 @pytest.mark.parametrize("M", [1, 15, 17, 96])
-@pytest.mark.parametrize("N,K,group", [(64, 256, 256), (512, 1280, 1280), (1280, 5120, 256), (960, 2816, 2816)])
+@pytest.mark.parametrize("N,K,group", [(64, 256, 256), (512, 1280, 1280), (1280, 5120, 256), (960, 2816, 2816),
+                                       (256, 256, 256), (1280, 512, 256), (512, 768, 768), (960, 768, 256)])
 def test_few_rows_same_bits_as_tiles(ext, M, N, K, group):
     """At most 96 rows take the few-row kernel (1 and 2 strips a workgroup, units that divide evenly over its waves and
-    not): dense, row-major 2:4 and stage-tiled 2:4, BIAS / RESID / GLU, per-row and grouped scales, with and without
+    not, fewer units than waves): dense, row-major 2:4 and stage-tiled 2:4, BIAS / RESID / GLU, per-row and grouped scales, with and without
     bias, equal the tile GEMM (a forced tile) bit for bit."""
     from kernels.cuda_ext import EPI_BIAS, EPI_GLU, EPI_RESID
     from kernels.fast_encoder import quantize_rows
