@@ -4,6 +4,7 @@
 #include "gemm_q8.h"
 #include "gemm_q8_rows.h"
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 
@@ -26,27 +27,28 @@ int num_cus() {
 
 // The time of a round of workgroups, one per CU, on each tile, in microseconds: c per 128-byte K stage, f for the launch,
 // the first stage and the epilogue, q8 for SILU_Q8's. 64x64 tiles (per_cu 2): two share a CU, each stage then taking
-// 1.3 times as long, and what is more than that counts by half rounds. (As whole rounds of two with one workgroup's
-// time, 7000 grouped rows x 1280 x 5120 took 64x64 tiles, 110 us, where 128x128 ones take 83.)
-// Fitted to graph replays of the encoder's linears at 376, 1892, 3000 and 8416 rows (K 1280 and 5120) and the bf16 stem,
-// cross-attention and layer shapes. Every tile timed for 18 linears (int8, 2:4, grouped, bf16) at 48 row counts from 6 to
-// 9024: the choice is within 4 % of the fastest tile at all but 19 of 849 points (18 of them bf16, the worst 1280 x 1280
-// over 7000 rows and more, 14 %) and EIGHT_WAVES' products, and nowhere slower than the former rule's beyond the noise.
-// Against that, the largest
-// tile that gives 64 % of the CUs a workgroup (the former rule): bf16 1892 x 1280 x 5120 62.2 -> 39.1 us, 1892 x 5120 x
-// 1280 SILU 48.3 -> 39.7, 1892 x 1280 x 1280 21.4 -> 13.9, 3000 x 1024 x 1280 15.0 -> 12.6; int8 3000 x 1280 x 1280 12.2
-// -> 9.5, grouped 1892 x 1280 x 5120 42.7 -> 28.3.
+// 1.25 to 1.35 times as long (the more, the more CUs hold two), and what is more than that counts by half rounds. (As
+// whole rounds of two with one workgroup's time, 7000 grouped rows x 1280 x 5120 took 64x64 tiles, 110 us, where 128x128
+// ones take 83.)
+// Fitted to graph replays of every tile at 889 products of each kind (int8; 2:4 row-major and stage-tiled; bf16; 781 with
+// grouped scales): 100 to 9024 rows, N 256 to 8192, K 256 to 5120, the encoder's, the stem's and the caches' among them.
+// The choice is within 4 % of the fastest tile at all but 8 stage-tiled, 9 row-major, 6 bf16 and 1 grouped of them, int8
+// aside (EIGHT_WAVES). Against the largest tile that gives 64 % of the CUs a workgroup (the former rule), 5245 products,
+// half of them of other sizes than the fit's (111 to 8000 rows, N 320 to 6144, K 640 to 3072), take 0.96 of the time on
+// average; 5 take more than 1.05 times it, at most 1.08. Some: bf16 1892 x 1280 x 5120 62.2 -> 39.1 us, 1892 x 5120 x 1280
+// SILU 48.3 -> 39.7, 1892 x 1280 x 1280 21.4 -> 13.9, 3000 x 1024 x 1280 15.0 -> 12.6; int8 3000 x 1280 x 1280 12.2 -> 9.5,
+// grouped 1892 x 1280 x 5120 42.7 -> 28.3.
 struct TileCost {
   int id;
   int per_cu;
   double c, f, q8;
 };
 constexpr TileCost BF16_COST[] = {{6, 1, 1.28, 10.9, 0.0}, {15, 1, 1.335, 10.0, 0.0}, {8, 1, .695, 7.5, 0.0},
-                                  {9, 1, .69, 6.6, 0.0},   {17, 1, .42, 4.5, 0.0},    {3, 1, .353, 3.3, 0.0},
+                                  {9, 1, .69, 6.6, 0.0},   {17, 1, .42, 4.5, 0.0},    {3, 1, .325, 4.1, 0.0},
                                   {7, 2, .265, 3.0, 0.0}};
 constexpr TileCost DENSE_COST[] = {{6, 1, 1.28, 10.9, 8.0}, {15, 1, 1.285, 10.5, 6.2}, {8, 1, .695, 7.5, 3.0},
-                                   {9, 1, .69, 6.6, 3.0},   {17, 1, .42, 4.5, 2.0},    {4, 1, .6, 4.0, 3.3},
-                                   {3, 1, .335, 3.3, 2.0},  {5, 1, .27, 3.1, 2.0},     {7, 2, .265, 3.0, 2.0}};
+                                   {9, 1, .69, 6.6, 3.0},   {17, 1, .42, 4.5, 2.0},    {4, 1, .6, 4.2, 3.3},
+                                   {3, 1, .335, 3.3, 2.0},  {5, 1, .27, 3.1, 2.0},     {7, 2, .268, 3.0, 2.0}};
 // int8 over several rounds: alone the 8-wave tiles (doubled fragments) are up to 10 % faster than 256x256 on 16 waves, but
 // whole layers that ran on them were up to 4 % slower, kernels that had not changed among them (2 blocks of 16 clips of
 // 200 to 376 frames 835 -> 860 us, of 24 x 376 1356 -> 1378; the attention 40.7 -> 44.9, the depthwise convolution 18.6 ->
@@ -55,14 +57,22 @@ constexpr TileCost DENSE_COST[] = {{6, 1, 1.28, 10.9, 8.0}, {15, 1, 1.285, 10.5,
 // us against 632 on one, and on another 666 where the former rule took 657. (Over one round they stay: 8 x 375 frames
 // 522 -> 509. bf16 layers gained at every size.)
 constexpr double EIGHT_WAVES = 1.25;
-// 2:4 weights; 10 reads stage-tiled records (row-major ones take 15)
-constexpr TileCost SPARSE_COST[] = {{10, 1, 1.03, 11.2, 7.0}, {15, 1, 1.25, 11.0, 7.0}, {8, 1, .58, 6.2, 3.5},
-                                    {9, 1, .52, 6.7, 3.5},    {17, 1, .47, 2.6, 2.0},   {0, 1, .437, 3.6, 2.0},
-                                    {4, 1, .447, 3.4, 4.1},   {3, 1, .315, 3.3, 2.0},   {5, 1, .27, 3.1, 2.0},
-                                    {7, 2, .25, 3.0, 2.0}};
+// stage-tiled 2:4 weights
+constexpr TileCost SPARSE_COST[] = {{10, 1, .902, 9.5, 7.0}, {15, 1, 1.25, 11.0, 7.0}, {8, 1, .589, 5.5, 3.5},
+                                    {9, 1, .442, 6.5, 3.5},  {17, 1, .555, 2.76, 2.0}, {0, 1, .409, 4.25, 2.0},
+                                    {4, 1, .492, 3.4, 4.1},  {3, 1, .296, 3.3, 2.0},   {5, 1, .27, 2.9, 2.0},
+                                    {7, 2, .2425, 3.0, 2.0}};
+// row-major 2:4 weights: 16 waves of 256x256 lose little to them, the 8-wave tiles over a long K much (with the tiled
+// weights' costs 3000 x 4096 x 4096 went to 128x256 tiles, 54 us, where 256x256 take 42)
+constexpr TileCost SPARSE_ROWS_COST[] = {{15, 1, .85, 9.9, 7.0},  {8, 1, .522, 5.83, 3.5}, {9, 1, .52, 6.7, 3.5},
+                                         {17, 1, .435, 3.4, 2.0}, {0, 1, .437, 3.6, 2.0},  {4, 1, .447, 3.4, 4.1},
+                                         {3, 1, .268, 3.5, 2.0},  {5, 1, .27, 2.9, 2.0},   {7, 2, .25, 3.0, 2.0}};
 // grouped scales (each group's fold is most of a stage); the larger 8-wave tiles spill
 constexpr TileCost GROUPED_COST[] = {{17, 1, .62, 3.6, 2.0}, {4, 1, .75, 3.5, 3.3},  {3, 1, .47, 3.4, 2.0},
                                      {5, 1, .35, 3.1, 2.0},  {7, 2, .34, 3.0, 2.0}};
+// and row-major 2:4 weights (3000 x 640 x 5120 64x64 tiles 24.9 us, 64x128 22.9)
+constexpr TileCost GROUPED_ROWS_COST[] = {{17, 1, .62, 3.6, 2.0},  {4, 1, .75, 3.5, 3.3}, {3, 1, .44, 3.5, 2.0},
+                                          {5, 1, .35, 3.1, 2.0},   {7, 2, .34, 3.0, 2.0}};
 
 int choose_tile(const GemmArgs& p, bool grouped, bool bf = false) {
   auto fits = [&](int id) {
@@ -83,16 +93,19 @@ int choose_tile(const GemmArgs& p, bool grouped, bool bf = false) {
   const bool dense = !grouped && !p.E && !bf;
   auto consider = [&](const auto& table) {
     for (const TileCost& t : table) {
-      if (!fits(t.id) || (p.E && !p.tiled && t.id == 10)) continue;
+      if (!fits(t.id)) continue;
       const int64_t n = (int64_t)((p.M + TILES[t.id].bm - 1) / TILES[t.id].bm) * (p.N / TILES[t.id].bn);
       const double rounds = (double)((n + cus - 1) / cus), once = t.f + (p.epi == EPI_SILU_Q8 ? t.q8 : 0.0);
       double us = t.per_cu == 1 || n <= cus ? rounds * (t.c * stages + once)
-                                            : rounds / 2 * (1.3 * t.c * stages + once);
+                                            : rounds / 2 * ((1.25 + .1 * std::min(1.0, (n - cus) / (double)cus)) *
+                                                                t.c * stages + once);
       if (dense && n > cus && (t.id == 8 || t.id == 9 || t.id == 17)) us *= EIGHT_WAVES;
       if (best < 0 || us < least) best = t.id, least = us;
     }
   };
-  if (grouped) consider(GROUPED_COST);
+  const bool rows24 = p.E && !p.tiled;
+  if (grouped) rows24 ? consider(GROUPED_ROWS_COST) : consider(GROUPED_COST);
+  else if (rows24) consider(SPARSE_ROWS_COST);
   else if (p.E) consider(SPARSE_COST);
   else if (bf) consider(BF16_COST);
   else consider(DENSE_COST);

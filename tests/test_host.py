@@ -191,6 +191,10 @@ def test_pack_24_tiled_matches_c_abi_and_round_trips():
     (0, 4, 8401, 2560, 1280, 1280, 15),  # several rounds, int8: whole layers are faster on 256x256
     (0, 0, 4601, 3840, 1280, 1280, 15), (0, 5, 4601, 5120, 1280, 1280, 15),  # 2 blocks 836 us, on 128x256 860
     (0, 4, 3000, 2560, 1280, 1280, 9),   # one round: 13.4, 17.4
+    (1, 0, 3000, 4096, 4096, 4096, 15), (1, 0, 8401, 1280, 5120, 5120, 15),  # row-major 2:4: 42 us, 128x256 54; 52, 72
+    (2, 0, 1500, 3840, 256, 256, 8),     # 8.1, 128x128 10.2
+    (1, 3, 3000, 640, 5120, 256, 3),     # 22.9, 64x64 24.9
+    (3, 0, 3000, 640, 5120, 5120, 3), (3, 0, 200, 5120, 5120, 5120, 7),  # 32.4, 35.7; 29.9, 31.2
     (2, 3, 376, 1280, 5120, 256, 7), (2, 5, 3000, 5120, 1280, 1280, 10), (4, 8, 3000, 16384, 1024, 1024, 15)])
 def test_gemm_tile_choice(kind, epi, M, N, K, group, tile):
     """The tile the cost model picks where another one was measured slower (microseconds beside the sizes)."""
