@@ -49,7 +49,7 @@ constexpr TileCost BF16_COST[] = {{6, 1, 1.28, 10.9, 0.0}, {15, 1, 1.335, 10.0, 
 constexpr TileCost DENSE_COST[] = {{6, 1, 1.28, 10.9, 8.0}, {15, 1, 1.285, 10.5, 6.2}, {8, 1, .695, 7.5, 3.0},
                                    {9, 1, .69, 6.6, 3.0},   {17, 1, .42, 4.5, 2.0},    {4, 1, .6, 4.2, 3.3},
                                    {3, 1, .335, 3.3, 2.0},  {5, 1, .27, 3.1, 2.0},     {7, 2, .268, 3.0, 2.0}};
-// int8 over several rounds: alone the 8-wave tiles (doubled fragments) are up to 10 % faster than 256x256 on 16 waves, but
+// int8 over several rounds: alone the 8-wave tiles (doubled fragments) are up to 18 % faster than 256x256 on 16 waves, but
 // whole layers that ran on them were up to 4 % slower, kernels that had not changed among them (2 blocks of 16 clips of
 // 200 to 376 frames 835 -> 860 us, of 24 x 376 1356 -> 1378; the attention 40.7 -> 44.9, the depthwise convolution 18.6 ->
 // 19.2): the chip's clock falls under the denser matrix work. Counted a quarter longer such products keep the 256x256
